@@ -269,3 +269,45 @@ def test_random_rows_positions_and_groups(cuda, seed):
     dev = Device(case, cuda, tokens)
     _step(case, dev, cuda, slots, lengths, tokens, dim ** -0.5)
     _step(case, dev, cuda, slots, None, tokens, dim ** -0.5)
+
+
+@pytest.mark.parametrize("rows,hq,hkv,dim,budget,dtype", [
+    (20, 32, 4, 128, 2048, torch.bfloat16),  # 640 spans: just above one round of one-shot workgroups
+    (33, 8, 8, 64, 2304, torch.float16),  # one query head per KV head
+    (9, 64, 2, 256, 1100, torch.bfloat16),  # two query blocks, a last span that is not whole
+    (48, 12, 2, 128, 1536, torch.float16),  # groups of 6
+])
+def test_streamed_batches(cuda, rows, hq, hkv, dim, budget, dtype):
+    """Batches of more than one round of spans (attention_stream_kernel): rows that end at and
+    beside step (128) and span (256) boundaries, empty and full rows, padding rows; one step
+    with device positions, two that read the working lengths.  A slot out of range zeroes its
+    row only."""
+    from ds355 import attention
+
+    case = Case(rows * 7 + dim, rows + 2, hkv, hq, dim, budget, dtype)
+    edges = [0, 1, 31, 32, 127, 128, 129, 255, 256, 257, 383, 384, 1000, budget - 4, budget - 5]
+    slots = [(5 * r + 3) % (rows + 2) if (rows + 2) % 5 else rows + 1 - r for r in range(rows)]
+    lengths = [min(edges[r % len(edges)], budget - 4) for r in range(rows)]
+    for s, n in zip(slots, lengths):
+        case.fill(s, n)
+    dev = Device(case, cuda, rows)
+    _step(case, dev, cuda, slots, lengths, rows + 2, dim ** -0.5, device_positions=True)
+    for _ in range(2):
+        _step(case, dev, cuda, slots, None, rows + 2, dim ** -0.5)
+    assert attention.attention_epoch(dev.ws) == 3
+    # One row's slot is out of range: zeros for it, the others as before.
+    q, k, v = case.inputs(rows)
+    outs = []
+    for bad in (None, rows // 2):
+        k_dev, v_dev, lens = dev.k.clone(), dev.v.clone(), dev.lens.clone()
+        out = torch.full_like(q, float("nan")).to(cuda)
+        chosen = [-1 if r == bad else s for r, s in enumerate(slots)]
+        attention.draft_linear_attention(q.to(cuda), k.to(cuda), v.to(cuda), out, k_dev, v_dev, lens, chosen, None,
+                                         scale=dim ** -0.5, workspace=dev.ws)
+        outs.append((out.cpu(), k_dev.cpu(), v_dev.cpu()))
+    keep = [r for r in range(rows) if r != rows // 2]
+    (whole, k_all, v_all), (partly, _, _) = outs
+    assert partly[rows // 2].count_nonzero() == 0
+    terms = attention_terms(q, k_all, v_all, slots, [n + 3 for n in lengths], dim ** -0.5)
+    assert_attention_close(partly[keep], whole[keep], terms[keep])  # other range ends: sums in another order
+    assert attention.attention_status(dev.ws) == attention.STATUS_BAD_POSITION

@@ -9,8 +9,9 @@
 //   out[r, h] = softmax(scale * q[r, h] . K[s, h / G, 0..p]) V[s, h / G, 0..p]
 // in fp32, and out rows past the batch are zero.
 //
-// Work split: one workgroup per (row, KV head, block of up to 16 query heads
-// of that KV head's group, span of tokens).  Each of its 4 waves walks
+// Work split (draft_attention_kernel; larger batches run
+// attention_stream_kernel, see there): one workgroup per (row, KV head, block
+// of up to 16 query heads of that KV head's group, span of tokens).  Each of its 4 waves walks
 // 16-token tiles of its quarter of the span:
 //   scores  S[t][g] = K[t] . Q[g]     one 16x16x32 bf16/fp16 MFMA per 32 of
 //                                     head_dim, K as the A operand (lane owns
@@ -56,6 +57,7 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -183,6 +185,25 @@ __device__ __forceinline__ f32x4 load16_sc1(Rsrc16 r, uint32_t off) {
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, kPolicySc1));
 }
 
+__device__ __forceinline__ f32x2 load8_sc1(Rsrc16 r, uint32_t off) {
+  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(off), 0, kPolicySc1));
+}
+
+// J consecutive 16-bit elements through a buffer resource.
+template <int J>
+__device__ __forceinline__ void load_words_buf(Rsrc16 r, int voff, int soff, uint32_t (&w)[J / 2]) {
+  if constexpr (J == 4) {
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    w[0] = v.x; w[1] = v.y;
+  } else {
+#pragma unroll
+    for (int h = 0; h < J / 8; ++h) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * h, soff, 0);
+      w[4 * h] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
+    }
+  }
+}
+
 __device__ __forceinline__ uint64_t tagged(uint32_t tag, float v) {
   return (static_cast<uint64_t>(tag) << 32) | __float_as_uint(v);
 }
@@ -221,13 +242,273 @@ __device__ __forceinline__ void zero_heads(const AttnArgs& a, int row, int head0
   }
 }
 
+// A wave's 32 tokens (two 16-token tiles): K rows for the score MFMAs, V rows
+// for the output.
+template <int D>
+struct KTiles {
+  u32x4 k[2][AttnShape<D>::kSteps];
+};
+template <int D>
+struct VTiles {
+  uint32_t v[2][4][AttnShape<D>::kJ / 2];
+};
+
+// A wave's running softmax state: lane (quad, col) holds query col's max and
+// sum (the sum over its own rows only) and D / 4 unnormalised outputs.
+template <int D>
+struct Running {
+  f32x4 acc[AttnShape<D>::kJ];
+  float m, l;
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int j = 0; j < AttnShape<D>::kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m = -INFINITY;
+    l = 0.f;
+  }
+};
+
+// Scores of the wave's 32 tokens: lane (quad, col) holds query col's scores
+// of tokens 4 * quad + i of each tile.
+template <int DT, int D>
+__device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv)[AttnShape<D>::kSteps],
+                                            f32x4 (&sc)[2]) {
+  sc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  sc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < AttnShape<D>::kSteps; ++i) {
+    sc[0] = mfma_scores<DT>(T.k[0][i], qv[i], sc[0]);
+    sc[1] = mfma_scores<DT>(T.k[1][i], qv[i], sc[1]);
+  }
+}
+
+// Online softmax and output of the 32 tokens tb .. tb + 31 (n valid tokens in
+// all).  The output MFMAs are 16x16x32 in the cache dtype with A = V^T and
+// B = P^T: k-slot (lane / 16, e) is token 4 * (lane / 16) + (e & 3) of tile
+// e / 4, i.e. the rows of the lane's own score tiles, and head_dim column m of
+// block j is d = J * m + j, so both operands are in the lane's registers.  P
+// is split into an upper part (its fp32 value cut to the dtype) and the dtype
+// rounding of the exact remainder; two MFMAs per block keep the products
+// within ~2^-16 of fp32 probabilities.
+template <int DT, int D>
+__device__ __forceinline__ void pair_output(const VTiles<D>& T, const f32x4 (&sc)[2], Running<D>& run, int tb, int n,
+                                            int quad, float c) {
+  constexpr int J = AttnShape<D>::kJ;
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = (tb + 4 * quad + i < n) ? sc[0][i] * c : -INFINITY;
+    x[4 + i] = (tb + kTileT + 4 * quad + i < n) ? sc[1][i] * c : -INFINITY;
+  }
+  float tmax = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+  tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+  tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+  const float mn = fmaxf(run.m, tmax);
+  const float alpha = fast_exp2(run.m - mn);
+  float p[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) p[e] = fast_exp2(x[e] - mn);
+  run.l = run.l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+  run.m = mn;
+#pragma unroll
+  for (int j = 0; j < J; ++j) run.acc[j] *= alpha;
+  u32x4 phi, plo;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t h0, h1, l0, l1;
+    split_prob<DT>(p[2 * w], h0, l0);
+    split_prob<DT>(p[2 * w + 1], h1, l1);
+    phi[w] = h0 | (h1 << 16);
+    plo[w] = l0 | (l1 << 16);
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low halves
+    const int w = j >> 1;
+    u32x4 av;
+    av[0] = __builtin_amdgcn_perm(T.v[0][1][w], T.v[0][0][w], sel);
+    av[1] = __builtin_amdgcn_perm(T.v[0][3][w], T.v[0][2][w], sel);
+    av[2] = __builtin_amdgcn_perm(T.v[1][1][w], T.v[1][0][w], sel);
+    av[3] = __builtin_amdgcn_perm(T.v[1][3][w], T.v[1][2][w], sel);
+    run.acc[j] = mfma_scores<DT>(av, phi, run.acc[j]);
+    run.acc[j] = mfma_scores<DT>(av, plo, run.acc[j]);
+  }
+}
+
+// LDS of one workgroup's merge: the waves' running max, sum and unnormalised
+// outputs.
+template <int D>
+struct MergeShared {
+  alignas(16) float acc[kWavesA][kGroupQ][D + 4];
+  float m[kWavesA][kGroupQ];
+  float l[kWavesA][kGroupQ];
+};
+
+// The waves' states go to LDS as they are (then a barrier).
+template <int D>
+__device__ __forceinline__ void waves_to_lds(MergeShared<D>& sh, const Running<D>& run, int wave, int quad, int col) {
+  constexpr int J = AttnShape<D>::kJ;
+  float l = run.l;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  const int d0 = 4 * J * quad;  // lane's outputs: d = d0 + J * i + j
+  if (quad == 0) {
+    sh.m[wave][col] = run.m;
+    sh.l[wave][col] = l;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) sh.acc[wave][col][d0 + J * i + j] = run.acc[j][i];
+  }
+}
+
+// The workgroup's (max, sum, outputs e .. e + 3) of query g: the waves in
+// wave order, common max, rescaled sums.
+template <int D>
+__device__ __forceinline__ f32x4 span_item(const MergeShared<D>& sh, int g, int e, float& mx, float& total_l) {
+  mx = sh.m[0][g];
+#pragma unroll
+  for (int w = 1; w < kWavesA; ++w) mx = fmaxf(mx, sh.m[w][g]);
+  total_l = 0.f;
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kWavesA; ++w) {
+    const float f = fast_exp2(sh.m[w][g] - mx);
+    total_l += sh.l[w][g] * f;
+    const f32x4 x = *reinterpret_cast<const f32x4*>(&sh.acc[w][g][e]);
+    v = w == 0 ? x * f : v + x * f;
+  }
+  return v;
+}
+
+template <int DT>
+__device__ __forceinline__ void store_out(const AttnArgs& a, int row, int head, int e, f32x4 v, float inv) {
+  uint16_t* o = static_cast<uint16_t*>(a.out) + row * a.o_row + head * a.o_head + e;
+  const uint32_t w0 = static_cast<uint32_t>(Elem<DT>::store(v[0] * inv)) |
+                      (static_cast<uint32_t>(Elem<DT>::store(v[1] * inv)) << 16);
+  const uint32_t w1 = static_cast<uint32_t>(Elem<DT>::store(v[2] * inv)) |
+                      (static_cast<uint32_t>(Elem<DT>::store(v[3] * inv)) << 16);
+  *reinterpret_cast<u32x2*>(o) = u32x2{w0, w1};
+}
+
+// The workgroup's result of `gcount` queries, written out normalised.
+template <int DT, int D>
+__device__ __forceinline__ void write_outputs(const AttnArgs& a, const MergeShared<D>& sh, int row, int head0,
+                                              int gcount, int tid) {
+  constexpr int kChunks = D / 4;
+  for (int item = tid; item < gcount * kChunks; item += kThreadsA) {
+    const int g = item / kChunks, e = 4 * (item % kChunks);
+    float mx, total_l;
+    const f32x4 v = span_item<D>(sh, g, e, mx, total_l);
+    store_out<DT>(a, row, head0 + g, e, v, 1.f / total_l);
+  }
+}
+
+// A unit done by several workgroups: this one's partial ((running max, sum,
+// unnormalised output) per query, fp32) goes to its place `off` (bytes) of
+// the partials with device-scope stores, which are waited for; then the
+// workgroup counts itself on the unit's counter.  True for the one that
+// counts last of `parts`: the others' stores are complete before their
+// counts, so it can read them without waiting, and it resets the counter for
+// the next launch.
+template <int D>
+__device__ __forceinline__ bool count_partial(const AttnArgs& a, const MergeShared<D>& sh, Rsrc16 prs, uint32_t off,
+                                              int gcount, int unit, int parts, int* s_last, int tid) {
+  using S = AttnShape<D>;
+  constexpr int kChunks = D / 4;
+  // Row g of a partial: D outputs, then (max, sum, 0, 0).
+  for (int item = tid; item < gcount * kChunks; item += kThreadsA) {
+    const int g = item / kChunks, e = 4 * (item % kChunks);
+    float mx, total_l;
+    const f32x4 v = span_item<D>(sh, g, e, mx, total_l);
+    store16_sc1(prs, off + static_cast<uint32_t>((g * S::kRow + e) * 4), v);
+    if (e == 0) store16_sc1(prs, off + static_cast<uint32_t>((g * S::kRow + D) * 4), f32x4{mx, total_l, 0.f, 0.f});
+  }
+  // Device-scope write-throughs: once this thread's are acknowledged they are
+  // visible to every workgroup.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t prev =
+        __hip_atomic_fetch_add(a.counters + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *s_last = prev == static_cast<uint32_t>(parts - 1) ? 1 : 0;
+    if (*s_last) coherent_store(a.counters + unit, 0u);
+  }
+  lds_barrier();
+  return *s_last != 0;
+}
+
+// Merge of a unit's `parts` partials in index order (so the result does not
+// depend on arrival order); part i is at place_of(i) (bytes), part `own` is
+// this workgroup's, taken from LDS.  The others' words of kGroupS parts are
+// requested at once.
+template <int DT, int D, typename PlaceOf>
+__device__ __forceinline__ void merge_partials(const AttnArgs& a, const MergeShared<D>& sh, Rsrc16 prs, int row,
+                                               int head0, int gcount, int parts, int own, int tid, PlaceOf place_of) {
+  using S = AttnShape<D>;
+  constexpr int kChunks = D / 4;
+  for (int item = tid; item < gcount * kChunks; item += kThreadsA) {
+    const int g = item / kChunks;
+    const int e = 4 * (item % kChunks);
+    float run_m = -INFINITY, run_l = 0.f;
+    f32x4 run = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < parts; s0 += kGroupS) {
+      const int cnt = min(kGroupS, parts - s0);
+      f32x4 pv[kGroupS];
+      f32x2 pml[kGroupS];
+#pragma unroll
+      for (int u = 0; u < kGroupS; ++u) {
+        const int sp = s0 + u;
+        if (u < cnt && sp != own) {
+          const uint32_t row_off = place_of(sp) + static_cast<uint32_t>(g * S::kRow * 4);
+          pv[u] = load16_sc1(prs, row_off + e * 4);
+          pml[u] = load8_sc1(prs, row_off + D * 4);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kGroupS; ++u) {
+        const int sp = s0 + u;
+        if (u >= cnt) break;
+        float m_s, l_s;
+        f32x4 a_s;
+        if (sp == own) {
+          a_s = span_item<D>(sh, g, e, m_s, l_s);
+        } else {
+          m_s = pml[u][0];
+          l_s = pml[u][1];
+          a_s = pv[u];
+        }
+        const float gm = fmaxf(run_m, m_s);
+        const float r1 = fast_exp2(run_m - gm);
+        const float r2 = fast_exp2(m_s - gm);
+        run_l = run_l * r1 + l_s * r2;
+        run = run * r1 + a_s * r2;
+        run_m = gm;
+      }
+    }
+    store_out<DT>(a, row, head0 + g, e, run, 1.f / run_l);
+  }
+}
+
+// The new token's K/V rows of one (row, KV head) go into the working cache
+// (workgroups of this launch read the input rows in their place).
+template <int D>
+__device__ __forceinline__ void write_token(const AttnArgs& a, int64_t work_base, int pos, const uint16_t* kin,
+                                            const uint16_t* vin, int tid) {
+  if (tid < D / 4) {
+    const int e = tid % (D / 8);
+    const bool is_v = tid >= D / 8;
+    uint16_t* dst = static_cast<uint16_t*>(is_v ? a.work_v : a.work_k) + work_base + static_cast<int64_t>(pos) * D;
+    *reinterpret_cast<u32x4*>(dst + 8 * e) = load16((is_v ? vin : kin) + 8 * e);
+  }
+}
+
 // Run by the grid's last workgroup at its end: once every workgroup of the
 // pending rows has stored its seen word (all of them have lower indices and
 // were dispatched before this one), each row's working length becomes
 // position + 1 and the epoch advances.
-__device__ __forceinline__ void publish(const AttnArgs& a, uint32_t tag) {
+__device__ __forceinline__ void publish(const AttnArgs& a, uint32_t tag, int seen_words) {
   bool expired = false;
-  const int seen_words = a.rows * a.hkv * a.qblocks * a.splits;
   for (int b = threadIdx.x; b < seen_words; b += kThreadsA) {
     if (b != static_cast<int>(blockIdx.x)) settle(a, a.seen + b, coherent_load(a.seen + b), tag, expired);
   }
@@ -246,9 +527,7 @@ template <int DT, int D>
 __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs a) {
   using S = AttnShape<D>;
   constexpr int J = S::kJ;
-  __shared__ float s_m[kWavesA][kGroupQ];
-  __shared__ float s_l[kWavesA][kGroupQ];
-  __shared__ float s_acc[kWavesA][kGroupQ][D + 4];
+  __shared__ MergeShared<D> sh;
   __shared__ int s_last;
   __shared__ int s_pos;
   __shared__ uint32_t s_tag;
@@ -293,33 +572,32 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   const uint16_t* vin = static_cast<const uint16_t*>(a.v_in) + row * a.v_row + kvh * a.v_head;
   const int t0 = split * S::kSpan + wave * S::kTiles * kTileT;
 
-  // One tile's operands: K rows for the score MFMAs, V rows for the output.
-  struct Tile {
-    u32x4 k[S::kSteps];
-    uint32_t v[4][J / 2];
-  };
-  // Loads of tile tb from the working rows only (rows clamped to the
+  // Loads of the 32 tokens from tb on, from the working rows only (rows clamped to the
   // cache); the rows from the position on are fixed up once it is known.
-  auto load_tile_rows = [&](Tile& T, int tb) {
-    const uint16_t* pk = kw + static_cast<int64_t>(min(tb + col, a.budget - 1)) * D + 8 * quad;
+  auto load_rows = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
-    for (int i = 0; i < S::kSteps; ++i) T.k[i] = load16(pk + 32 * i);
+    for (int h = 0; h < 2; ++h) {
+      const uint16_t* pk = kw + static_cast<int64_t>(min(tb + h * kTileT + col, a.budget - 1)) * D + 8 * quad;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      load_words<J>(vw + static_cast<int64_t>(min(tb + 4 * quad + r, a.budget - 1)) * D + J * col, T.v[r]);
+      for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = load16(pk + 32 * i);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        load_words<J>(vw + static_cast<int64_t>(min(tb + h * kTileT + 4 * quad + r, a.budget - 1)) * D + J * col,
+                      V.v[h][r]);
+      }
     }
   };
   // The first pair of the wave's tiles and this row's input K / V slices are
   // requested before the position arrives (the position is a second
   // dependent load after the slot).  Every address is valid whatever the
   // position: working rows below the cache capacity and the input row.
-  Tile ta, tb_, tc, td;
+  KTiles<D> k0, k1;
+  VTiles<D> v0, v1;
   u32x4 kin_s[S::kSteps];
   uint32_t vin_s[J / 2];
   const bool early = real && slot_ok && t0 < a.budget;
   if (early) {
-    load_tile_rows(ta, t0);
-    load_tile_rows(tb_, t0 + kTileT);
+    load_rows(k0, v0, t0);
 #pragma unroll
     for (int i = 0; i < S::kSteps; ++i) kin_s[i] = load16(kin + 8 * quad + 32 * i);
     load_words<J>(vin + J * col, vin_s);
@@ -331,7 +609,7 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   const int n = valid ? pos + 1 : 0;
   const int active = valid ? (n + S::kSpan - 1) / S::kSpan : 1;
   auto finish = [&]() {
-    if (blockIdx.x == gridDim.x - 1) publish(a, tag);
+    if (blockIdx.x == gridDim.x - 1) publish(a, tag, a.rows * a.hkv * a.qblocks * a.splits);
   };
 
   if (!real) {  // padding row: zero once
@@ -365,10 +643,8 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
     }
   }
 
-  f32x4 acc[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, lsum = 0.f;
+  Running<D> run;
+  run.clear();
   const float c = a.scale * kLog2e;
 
   // Rows at or past n read row n - 1 = pos (the new token's input row): a
@@ -376,83 +652,39 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   auto row_ptr = [&](const uint16_t* work, const uint16_t* in, int t) {
     return t >= pos ? in : work + static_cast<int64_t>(t) * D;
   };
-  auto load_tile = [&](Tile& T, int tb) {
-    const uint16_t* pk = row_ptr(kw, kin, tb + col) + 8 * quad;
+  auto load_pair = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
-    for (int i = 0; i < S::kSteps; ++i) T.k[i] = load16(pk + 32 * i);
+    for (int h = 0; h < 2; ++h) {
+      const uint16_t* pk = row_ptr(kw, kin, tb + h * kTileT + col) + 8 * quad;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) load_words<J>(row_ptr(vw, vin, tb + 4 * quad + r) + J * col, T.v[r]);
+      for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = load16(pk + 32 * i);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) load_words<J>(row_ptr(vw, vin, tb + h * kTileT + 4 * quad + r) + J * col, V.v[h][r]);
+    }
   };
-  // A tile loaded from the working rows: the position's row becomes the
+  // A pair loaded from the working rows: the position's row becomes the
   // input row, later rows of V become zeros (their probabilities are 0, and
   // stale cache words may not be finite; K rows there only feed masked
   // scores).
-  auto fix_tile = [&](Tile& T, int tb) {
-    if (tb + col == pos) {
+  auto fix_pair = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
-      for (int i = 0; i < S::kSteps; ++i) T.k[i] = kin_s[i];
-    }
+    for (int h = 0; h < 2; ++h) {
+      if (tb + h * kTileT + col == pos) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = tb + 4 * quad + r;
+        for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = kin_s[i];
+      }
 #pragma unroll
-      for (int w = 0; w < J / 2; ++w) T.v[r][w] = t == pos ? vin_s[w] : (t > pos ? 0u : T.v[r][w]);
+      for (int r = 0; r < 4; ++r) {
+        const int t = tb + h * kTileT + 4 * quad + r;
+#pragma unroll
+        for (int w = 0; w < J / 2; ++w) V.v[h][r][w] = t == pos ? vin_s[w] : (t > pos ? 0u : V.v[h][r][w]);
+      }
     }
   };
-  // Scores, online softmax and output for the 32 tokens tb .. tb + 31 held in
-  // tiles T0 and T1.  The output MFMAs are 16x16x32 in the cache dtype with
-  // A = V^T and B = P^T: k-slot (lane / 16, e) is token 4 * (lane / 16) +
-  // (e & 3) of tile e / 4, i.e. the rows of the lane's own score tiles, and
-  // head_dim column m of block j is d = J * m + j, so both operands are in the
-  // lane's registers.  P is split into an upper part (its fp32 value cut to
-  // the dtype) and the dtype rounding of the exact remainder; two MFMAs per
-  // block keep the products within ~2^-16 of fp32 probabilities.
-  auto compute_pair = [&](const Tile& T0, const Tile& T1, int tb) {
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < S::kSteps; ++i) {
-      s0 = mfma_scores<DT>(T0.k[i], qv[i], s0);
-      s1 = mfma_scores<DT>(T1.k[i], qv[i], s1);
-    }
-    float x[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[i] = (tb + 4 * quad + i < n) ? s0[i] * c : -INFINITY;
-      x[4 + i] = (tb + kTileT + 4 * quad + i < n) ? s1[i] * c : -INFINITY;
-    }
-    float tmax = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float mn = fmaxf(m, tmax);
-    const float alpha = fast_exp2(m - mn);
-    float p[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) p[e] = fast_exp2(x[e] - mn);
-    lsum = lsum * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
-    m = mn;
-#pragma unroll
-    for (int j = 0; j < J; ++j) acc[j] *= alpha;
-    u32x4 phi, plo;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      uint32_t h0, h1, l0, l1;
-      split_prob<DT>(p[2 * w], h0, l0);
-      split_prob<DT>(p[2 * w + 1], h1, l1);
-      phi[w] = h0 | (h1 << 16);
-      plo[w] = l0 | (l1 << 16);
-    }
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low halves
-      const int w = j >> 1;
-      u32x4 av;
-      av[0] = __builtin_amdgcn_perm(T0.v[1][w], T0.v[0][w], sel);
-      av[1] = __builtin_amdgcn_perm(T0.v[3][w], T0.v[2][w], sel);
-      av[2] = __builtin_amdgcn_perm(T1.v[1][w], T1.v[0][w], sel);
-      av[3] = __builtin_amdgcn_perm(T1.v[3][w], T1.v[2][w], sel);
-      acc[j] = mfma_scores<DT>(av, phi, acc[j]);
-      acc[j] = mfma_scores<DT>(av, plo, acc[j]);
-    }
+  auto compute_pair = [&](const KTiles<D>& K, const VTiles<D>& V, int tb) {
+    f32x4 sc[2];
+    pair_scores<DT, D>(K, qv, sc);
+    pair_output<DT, D>(V, sc, run, tb, n, quad, c);
   };
 
   // The first pair came from the working rows and is fixed up here; the
@@ -461,167 +693,304 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   // their use); a pair wholly past n is loaded (cache hits on row pos) but
   // not computed.
   if (t0 < n) {
-    fix_tile(ta, t0);
-    fix_tile(tb_, t0 + kTileT);
+    fix_pair(k0, v0, t0);
     if constexpr (S::kTiles == 4) {
-      load_tile(tc, t0 + 2 * kTileT);
-      load_tile(td, t0 + 3 * kTileT);
+      load_pair(k1, v1, t0 + 2 * kTileT);
       __builtin_amdgcn_sched_barrier(0);
-      compute_pair(ta, tb_, t0);
-      if (t0 + 2 * kTileT < n) compute_pair(tc, td, t0 + 2 * kTileT);
+      compute_pair(k0, v0, t0);
+      if (t0 + 2 * kTileT < n) compute_pair(k1, v1, t0 + 2 * kTileT);
     } else {
-      compute_pair(ta, tb_, t0);
+      compute_pair(k0, v0, t0);
     }
   }
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
 
-  // The new token goes into the working cache (a workgroup of this launch
-  // that reads that row of the cache early replaces it with the input row).
-  if (qb == 0 && split == pos / S::kSpan && threadIdx.x < D / 4) {
-    const int e = threadIdx.x % (D / 8);
-    const bool is_v = threadIdx.x >= D / 8;
-    uint16_t* dst = static_cast<uint16_t*>(is_v ? a.work_v : a.work_k) + work_base + static_cast<int64_t>(pos) * D;
-    *reinterpret_cast<u32x4*>(dst + 8 * e) = load16((is_v ? vin : kin) + 8 * e);
-  }
-
-  // The four waves' running max, sum and unnormalised outputs go to LDS as
-  // they are; one barrier, then thread t merges item (query g, outputs e ..
-  // e + 3) over the waves in wave order: common max, rescaled sums.
-  const int d0 = 4 * J * quad;  // lane's outputs: d = d0 + J * i + j
-  if (quad == 0) {
-    s_m[wave][col] = m;
-    s_l[wave][col] = lsum;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) s_acc[wave][col][d0 + J * i + j] = acc[j][i];
-  }
+  if (qb == 0 && split == pos / S::kSpan) write_token<D>(a, work_base, pos, kin, vin, threadIdx.x);
+  waves_to_lds<D>(sh, run, wave, quad, col);
   lds_barrier();
-  constexpr int kChunks = D / 4;
-  const int items = gcount * kChunks;
-  // This span's (max, sum, outputs e .. e + 3) of query g.
-  auto span_item = [&](int g, int e, float& mx, float& total_l) -> f32x4 {
-    mx = s_m[0][g];
-#pragma unroll
-    for (int w = 1; w < kWavesA; ++w) mx = fmaxf(mx, s_m[w][g]);
-    total_l = 0.f;
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kWavesA; ++w) {
-      const float f = fast_exp2(s_m[w][g] - mx);
-      total_l += s_l[w][g] * f;
-      const f32x4 x = *reinterpret_cast<const f32x4*>(&s_acc[w][g][e]);
-      v = w == 0 ? x * f : v + x * f;
-    }
-    return v;
-  };
-  auto store_out = [&](int g, int e, f32x4 v, float inv) {
-    uint16_t* o = static_cast<uint16_t*>(a.out) + row * a.o_row + (head0 + g) * a.o_head + e;
-    const uint32_t w0 = static_cast<uint32_t>(Elem<DT>::store(v[0] * inv)) |
-                        (static_cast<uint32_t>(Elem<DT>::store(v[1] * inv)) << 16);
-    const uint32_t w1 = static_cast<uint32_t>(Elem<DT>::store(v[2] * inv)) |
-                        (static_cast<uint32_t>(Elem<DT>::store(v[3] * inv)) << 16);
-    *reinterpret_cast<u32x2*>(o) = u32x2{w0, w1};
-  };
-
   if (active == 1) {
-    for (int item = threadIdx.x; item < items; item += kThreadsA) {
-      const int g = item / kChunks, e = 4 * (item % kChunks);
-      float mx, total_l;
-      const f32x4 v = span_item(g, e, mx, total_l);
-      store_out(g, e, v, 1.f / total_l);
-    }
+    write_outputs<DT, D>(a, sh, row, head0, gcount, threadIdx.x);
     finish();
     return;
   }
 
-  // Several spans.  Every span writes its result ((running max, sum,
-  // unnormalised output) per query, fp32) to its slot of the row's partials
-  // with device-scope stores, waits until they are done and counts itself on
-  // the row's counter.  The workgroup that counts last merges the row: the
-  // others' stores are complete before their counts, so it reads them
-  // without waiting, and it resets the counter for the next launch.  The
-  // spans are merged in index order whichever workgroup merges, so the
-  // result does not depend on arrival order.
+  // Several spans: the one that counts last merges the row's partials.
   const int unit = (row * a.hkv + kvh) * a.qblocks + qb;
-  float* part_base = a.partials + static_cast<int64_t>(unit) * a.splits * kGroupQ * S::kRow;
-  // The row's partials as a buffer resource: 16-byte device-scope (sc1)
-  // accesses, written through to memory and read past the per-XCD caches.
-  const Rsrc16 prs = make_rsrc16(part_base, static_cast<int64_t>(a.splits) * kGroupQ * S::kRow * 4);
-  // Row g of a span's partial: D outputs, then (max, sum, 0, 0).
-  const uint32_t span_off = static_cast<uint32_t>(split * kGroupQ * S::kRow * 4);
-  for (int item = threadIdx.x; item < items; item += kThreadsA) {
-    const int g = item / kChunks, e = 4 * (item % kChunks);
-    float mx, total_l;
-    const f32x4 v = span_item(g, e, mx, total_l);
-    store16_sc1(prs, span_off + static_cast<uint32_t>((g * S::kRow + e) * 4), v);
-    if (e == 0) store16_sc1(prs, span_off + static_cast<uint32_t>((g * S::kRow + D) * 4), f32x4{mx, total_l, 0.f, 0.f});
-  }
-  // The stores are device-scope write-throughs: once this thread's are
-  // acknowledged they are visible to every workgroup.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t prev =
-        __hip_atomic_fetch_add(a.counters + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = prev == static_cast<uint32_t>(active - 1) ? 1 : 0;
-    if (s_last) coherent_store(a.counters + unit, 0u);
-  }
-  lds_barrier();
-  if (!s_last) {
-    finish();
-    return;
-  }
-
-  // Merge: spans in index order, every other span's words requested at once
-  // (kGroupS spans per round); this span's values come from LDS.
-  for (int item = threadIdx.x; item < items; item += kThreadsA) {
-    const int g = item / kChunks;
-    const int e = 4 * (item % kChunks);
-    float run_m = -INFINITY, run_l = 0.f;
-    f32x4 run = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < active; s0 += kGroupS) {
-      const int cnt = min(kGroupS, active - s0);
-      f32x4 pv[kGroupS], pml[kGroupS];
-#pragma unroll
-      for (int u = 0; u < kGroupS; ++u) {
-        const int sp = s0 + u;
-        if (u < cnt && sp != split) {
-          const uint32_t row_off = static_cast<uint32_t>((sp * kGroupQ + g) * S::kRow * 4);
-          pv[u] = load16_sc1(prs, row_off + e * 4);
-          pml[u] = load16_sc1(prs, row_off + D * 4);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kGroupS; ++u) {
-        const int sp = s0 + u;
-        if (u >= cnt) break;
-        float m_s, l_s;
-        f32x4 a_s;
-        if (sp == split) {
-          a_s = span_item(g, e, m_s, l_s);
-        } else {
-          m_s = pml[u][0];
-          l_s = pml[u][1];
-          a_s = pv[u];
-        }
-        const float gm = fmaxf(run_m, m_s);
-        const float r1 = fast_exp2(run_m - gm);
-        const float r2 = fast_exp2(m_s - gm);
-        run_l = run_l * r1 + l_s * r2;
-        run = run * r1 + a_s * r2;
-        run_m = gm;
-      }
-    }
-    store_out(g, e, run, 1.f / run_l);
+  constexpr int kPartBytes = kGroupQ * S::kRow * 4;
+  const Rsrc16 prs = make_rsrc16(a.partials + static_cast<int64_t>(unit) * a.splits * kGroupQ * S::kRow,
+                                 static_cast<int64_t>(a.splits) * kPartBytes);
+  if (count_partial<D>(a, sh, prs, static_cast<uint32_t>(split * kPartBytes), gcount, unit, active, &s_last,
+                       threadIdx.x)) {
+    merge_partials<DT, D>(a, sh, prs, row, head0, gcount, active, split, threadIdx.x,
+                          [](int sp) { return static_cast<uint32_t>(sp * kPartBytes); });
   }
   finish();
 }
 
+// ---- Batches of more than one round of spans --------------------------------
+// The same attention with the work dealt evenly.  Bound by HBM reads; one
+// workgroup per span lost to it on large batches: every workgroup pays its
+// own ramp, wave merge and partial, rows' empty spans are launched too, and
+// the last round of workgroups is partly empty.
+//   - The tokens of every (row, KV head, query block) unit are cut into steps
+//     of 128 (32 per wave); the steps of all units are numbered unit by unit
+//     (a prefix sum over the rows' positions, in LDS), and each resident
+//     workgroup takes one contiguous range, so all end together whatever the
+//     rows' lengths.
+//   - Within a unit a wave requests the next step's K as soon as the score
+//     MFMAs have read the current K, and the next V after the output MFMAs.
+//   - A unit inside one range is finished in place.  A unit cut by range
+//     ends is merged by the workgroup that counts last on it, partials in
+//     range order (the result does not depend on arrival).  A range has at
+//     most two cut units, its first and its last: two partial slots.
+// Fewer, longer ranges won: every unit boundary costs a merge and a cold
+// start, and 4 waves x 16 KB in flight per CU already fill the memory queue.
+// us on 57 rows of 300-3970 tokens (64/8 heads x 128, fp16) / 64 rows of 1987
+// (32/4 x 128) / 16 rows of 1984-3990 (32/8 x 256) / 48 rows of 984-1990
+// (32/8 x 64); bandwidth of the last line 5.0, 5.5, 5.0 and 4.4 TB/s:
+//   one workgroup per span                          184 / 63 / 130 / 43.5
+//   ranges, 3 workgroups per CU (2 at 256, 4 at 64) 118 / 64 / 121 / 38.0
+//   ranges, 2 (2, 3)                                106 / 52 / 121 / 37.6
+//   ranges, 1 (1, 2), kept                          107 / 48 /  82 / 34.8
+// (at 256 two per CU spill 42 registers).  Two steps in flight per wave: 110
+// / 48.6 / 82 / 35.5.  The next unit's operands requested before the merge:
+// 105 / 54 / 82 / 34.9, no gain for 35 more registers.
+template <int D>
+struct StreamShape {
+  static constexpr int kStep = kWavesA * 2 * kTileT;            // tokens per step (32 per wave)
+  static constexpr int kPerCu = D == 64 ? 2 : 1;       // workgroups per CU
+  // Spans above which the batch is streamed: about one round of one-shot
+  // workgroups (4 per CU at head_dim 64, 2 at 128).  us, one-shot against
+  // streamed, at 512 spans of head_dim 128: 16.6 / 17.2 (16 rows of 1987
+  // tokens), 14.4 / 17.2 (64 rows of 184-487); at 576: 21.0 / 20.4; at 768:
+  // 26.2 / 23.8 (1987 tokens), 18.9 / 13.8 (100-400).  Head_dim 64, 1024
+  // spans: 17.7 / 17.6 (32 x 1987), 14.6 / 16.2 (64 rows of 184-487).
+  // Head_dim 256, 256 spans 18.8 / 18.6, 512 spans 23.5 / 21.6.
+  static constexpr int kOneRound = D == 64 ? 1024 : (D == 128 ? 512 : 256);
+};
+constexpr int kMinSteps = 2;  // steps per workgroup, at least
+
+struct Steps {  // workgroup w < used takes steps [start(w), start(w + 1))
+  int base, rem, used;
+  __device__ __forceinline__ int start(int w) const { return w * base + min(w, rem); }
+  __device__ __forceinline__ int owner(int x) const {
+    const int wide = rem * (base + 1);
+    return __builtin_amdgcn_readfirstlane(x < wide ? x / (base + 1) : rem + (x - wide) / base);
+  }
+};
+
+template <int DT, int D>
+__global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_stream_kernel(AttnArgs a) {
+  using S = AttnShape<D>;
+  constexpr int J = S::kJ;
+  constexpr int kStep = StreamShape<D>::kStep;
+  __shared__ MergeShared<D> sh;
+  __shared__ int s_prefix[kMaxRows + 1];  // steps of one unit of each row, exclusive prefix
+  __shared__ int s_pos[kMaxRows];
+  __shared__ int s_slot[kMaxRows];
+  __shared__ int s_scratch[4];
+  __shared__ int s_last;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15;
+  const int quad = lane >> 4;
+  const int units_row = a.hkv * a.qblocks;
+
+  const uint32_t tag =
+      static_cast<uint32_t>(scalar_load(reinterpret_cast<const int32_t*>(a.header + kHdrEpoch))) + 1u;
+  build_row_prefix(a.rows, s_prefix, s_scratch, [&](int r) {
+    const int slot = a.slots[r];
+    int pos = -1;
+    if (slot >= 0 && slot < a.num_slots) pos = a.positions ? a.positions[r] : a.working_lens[slot];
+    if (pos >= a.budget) pos = -1;
+    s_pos[r] = max(pos, -1);
+    s_slot[r] = slot;
+    return pos >= 0 ? (pos + kStep) / kStep : 0;
+  });
+  // Every thread's reads of the positions and the epoch have landed (the
+  // prefix's barriers waited for them): the workgroup's seen word may go out.
+  if (threadIdx.x == 0 && a.rows > 0) coherent_store(a.seen + blockIdx.x, tagged(tag, 0.f));
+
+  // Padding rows and rows with a bad slot or position are zero.
+  for (int r = blockIdx.x; r < a.out_rows; r += gridDim.x) {
+    if (r >= a.rows || s_pos[r] < 0) zero_heads<D>(a, r, 0, a.hq);
+  }
+
+  const int total = __builtin_amdgcn_readfirstlane(s_prefix[a.rows]) * units_row;
+  Steps st;
+  st.used = min(static_cast<int>(gridDim.x), max(1, total / kMinSteps));
+  st.base = __builtin_amdgcn_readfirstlane(total / st.used);
+  st.rem = total - st.base * st.used;
+  const int w = blockIdx.x;
+  const int first = w < st.used ? st.start(w) : 0;
+  const int end = w < st.used ? st.start(w + 1) : 0;
+
+  // One unit: row, KV head, query block and its steps [s0, s0 + count).
+  struct Unit {
+    int row, kvh, qb, s0, count, pos;
+    int64_t work;  // element offset of the working rows
+  };
+  int row_hint = 0;
+  auto unit_at = [&](int s) {
+    int lo = row_hint, hi = a.rows - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s_prefix[mid] * units_row <= s) lo = mid; else hi = mid - 1;
+    }
+    Unit u;
+    u.row = __builtin_amdgcn_readfirstlane(lo);
+    row_hint = u.row;
+    u.pos = __builtin_amdgcn_readfirstlane(s_pos[u.row]);
+    u.count = (u.pos + kStep) / kStep;
+    const int base = __builtin_amdgcn_readfirstlane(s_prefix[u.row]) * units_row;
+    const int k = __builtin_amdgcn_readfirstlane((s - base) / u.count);
+    u.s0 = base + k * u.count;
+    u.kvh = __builtin_amdgcn_readfirstlane(k / a.qblocks);
+    u.qb = k - u.kvh * a.qblocks;
+    const int slot = __builtin_amdgcn_readfirstlane(s_slot[u.row]);
+    u.work = (static_cast<int64_t>(slot) * a.hkv + u.kvh) * a.budget * D;
+    // Made scalar: quotients are computed in vector registers, and a buffer
+    // resource held there costs a loop over the lanes at every load.
+    u.s0 = __builtin_amdgcn_readfirstlane(u.s0);
+    u.count = __builtin_amdgcn_readfirstlane(u.count);
+    u.qb = __builtin_amdgcn_readfirstlane(u.qb);
+    u.work = uniform64(u.work);
+    return u;
+  };
+  // This wave's 32 tokens of step s start at token_of(u, s).
+  auto token_of = [&](const Unit& u, int s) { return (s - u.s0) * kStep + wave * (kStep / kWavesA); };
+  auto kin_of = [&](const Unit& u) { return static_cast<const uint16_t*>(a.k_in) + u.row * a.k_row + u.kvh * a.k_head; };
+  auto vin_of = [&](const Unit& u) { return static_cast<const uint16_t*>(a.v_in) + u.row * a.v_row + u.kvh * a.v_head; };
+  // Loads of the 32 tokens from tb on: buffer loads from the unit's working
+  // rows (a scalar base, one lane offset, fixed steps).  Rows at or past the
+  // position come from the new token's input row instead (its scores past
+  // the position are masked): the unit's last waves choose per lane.
+  const int k_lane = (col * D + 8 * quad) * 2;
+  const int v_lane = (4 * quad * D + J * col) * 2;
+  const int unit_bytes = a.budget * D * 2;
+  auto load_k = [&](KTiles<D>& T, const Unit& u, int token) {
+    const int tb = __builtin_amdgcn_readfirstlane(token);
+    const uint16_t* rows_k = static_cast<const uint16_t*>(a.work_k) + uniform64(u.work);
+    if (tb + 2 * kTileT <= u.pos) {  // wave-uniform
+      const Rsrc16 r = make_rsrc16(rows_k, unit_bytes);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int at = (tb + h * kTileT) * D * 2;
+#pragma unroll
+        for (int i = 0; i < S::kSteps; ++i) {
+          T.k[h][i] = __builtin_amdgcn_raw_buffer_load_b128(r, k_lane + 64 * i, at, 0);
+        }
+      }
+    } else {
+      const uint16_t* in = kin_of(u);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int t = tb + h * kTileT + col;
+        const uint16_t* p = (t >= u.pos ? in : rows_k + static_cast<int64_t>(t) * D) + 8 * quad;
+#pragma unroll
+        for (int i = 0; i < S::kSteps; ++i) T.k[h][i] = load16(p + 32 * i);
+      }
+    }
+  };
+  auto load_v = [&](VTiles<D>& T, const Unit& u, int token) {
+    const int tb = __builtin_amdgcn_readfirstlane(token);
+    const uint16_t* rows_v = static_cast<const uint16_t*>(a.work_v) + uniform64(u.work);
+    if (tb + 2 * kTileT <= u.pos) {  // wave-uniform
+      const Rsrc16 rs = make_rsrc16(rows_v, unit_bytes);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) load_words_buf<J>(rs, v_lane + r * D * 2, (tb + h * kTileT) * D * 2, T.v[h][r]);
+      }
+    } else {
+      const uint16_t* in = vin_of(u);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = tb + h * kTileT + 4 * quad + r;
+          load_words<J>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + J * col, T.v[h][r]);
+        }
+      }
+    }
+  };
+  u32x4 qv[S::kSteps];
+  auto load_q = [&](const Unit& u) {
+    const int g0 = u.qb * kGroupQ, gcount = min(kGroupQ, a.group - g0);
+    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + u.row * a.q_row +
+                         (u.kvh * a.group + g0 + min(col, gcount - 1)) * a.q_head + 8 * quad;
+#pragma unroll
+    for (int i = 0; i < S::kSteps; ++i) {
+      const u32x4 v = load16(qp + 32 * i);
+      qv[i] = col < gcount ? v : u32x4{0, 0, 0, 0};
+    }
+  };
+
+  constexpr int kPartBytes = kGroupQ * S::kRow * 4;
+  const Rsrc16 prs = make_rsrc16(a.partials, static_cast<int64_t>(gridDim.x) * 2 * kPartBytes);
+  const float c = a.scale * kLog2e;
+  for (int s = first; s < end;) {
+    const Unit u = unit_at(s);
+    const int unit_end = u.s0 + u.count;
+    const int stop = min(unit_end, end);  // this range's steps of the unit: [s, stop)
+    const bool whole = s == u.s0 && stop == unit_end;
+    const int n = u.pos + 1;
+    KTiles<D> K;
+    VTiles<D> V;
+    Running<D> run;
+    run.clear();
+    load_q(u);
+    int tb = token_of(u, s);
+    load_k(K, u, tb);
+    load_v(V, u, tb);
+    for (;;) {
+      const bool more = ++s < stop;
+      f32x4 sc[2];
+      pair_scores<DT, D>(K, qv, sc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) load_k(K, u, tb + kStep);
+      __builtin_amdgcn_sched_barrier(0);
+      if (tb < n) pair_output<DT, D>(V, sc, run, tb, n, quad, c);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!more) break;
+      tb += kStep;
+      load_v(V, u, tb);
+    }
+    const int g0 = u.qb * kGroupQ, gcount = min(kGroupQ, a.group - g0);
+    const int head0 = u.kvh * a.group + g0;
+    if (u.qb == 0 && stop == unit_end) write_token<D>(a, u.work, u.pos, kin_of(u), vin_of(u), threadIdx.x);
+    waves_to_lds<D>(sh, run, wave, quad, col);
+    lds_barrier();
+    if (whole) {
+      write_outputs<DT, D>(a, sh, u.row, head0, gcount, threadIdx.x);
+    } else {
+      const int w0 = st.owner(u.s0);
+      const int parts = st.owner(unit_end - 1) - w0 + 1;
+      auto place_of = [&](int i) {  // slot 1 of a range that starts in an earlier unit, else slot 0
+        return static_cast<uint32_t>((2 * (w0 + i) + (st.start(w0 + i) < u.s0 ? 1 : 0)) * kPartBytes);
+      };
+      const int unit = (u.row * a.hkv + u.kvh) * a.qblocks + u.qb;
+      if (count_partial<D>(a, sh, prs, place_of(w - w0), gcount, unit, parts, &s_last, threadIdx.x)) {
+        merge_partials<DT, D>(a, sh, prs, u.row, head0, gcount, parts, w - w0, threadIdx.x, place_of);
+      }
+    }
+    lds_barrier();  // the next unit's states overwrite these
+  }
+  if (blockIdx.x == gridDim.x - 1) publish(a, tag, gridDim.x);
+}
+
 template <int DT, int D>
 int launch_attention(hipStream_t stream, const AttnArgs& a) {
+  const int64_t spans = static_cast<int64_t>(a.rows) * a.hkv * a.qblocks * a.splits;
+  const int64_t steps = static_cast<int64_t>(a.rows) * a.hkv * a.qblocks *
+                        ((a.budget + StreamShape<D>::kStep - 1) / StreamShape<D>::kStep);
+  // (32-bit step numbers and byte offsets within a unit's rows.)
+  if (spans > StreamShape<D>::kOneRound && steps < (int64_t{1} << 30) && static_cast<int64_t>(a.budget) * D * 2 < INT32_MAX) {
+    // Two partial slots per workgroup, out of the workspace's one per span.
+    const int64_t grid = std::min<int64_t>(static_cast<int64_t>(StreamShape<D>::kPerCu) * device_cu_count(), spans / 2);
+    attention_stream_kernel<DT, D><<<static_cast<unsigned>(grid), kThreadsA, 0, stream>>>(a);
+    return check_launch("ds_draft_attention");
+  }
   const int64_t grid = static_cast<int64_t>(a.out_rows) * a.hkv * a.qblocks * a.splits;
   draft_attention_kernel<DT, D><<<static_cast<unsigned>(grid), kThreadsA, 0, stream>>>(a);
   return check_launch("ds_draft_attention");
