@@ -70,6 +70,18 @@ def test_fused_pages_not_a_power_of_two(cuda, seed, kw):
     _same(chain, fused)
 
 
+@pytest.mark.parametrize("rows,lse", [(9, True), (40, True), (70, True), (40, False)])
+def test_fused_short_rows_more_selectors(cuda, rows, lse):
+    """Short rows: a selector per row, up to 64 of them (70 rows: some take two), instead of 8.
+    The chain's bytes, and (with an LSE) oracle parity."""
+    case = _ragged(50 + rows, rows, 1, 1800, hkv=2, hq=16, head_dim=64, chunk=32, token_budget=1024)
+    fused = run_gpu(case, cuda, path="fused", lse_free=not lse)
+    if lse:
+        check_step(case, fused)
+    chain = run_gpu(case, cuda, path="chain", lse_free=not lse)
+    _same(chain, fused, KEYS if lse else LSE_FREE_KEYS)
+
+
 def test_fused_repeated_launches_and_reused_workspace(cuda):
     """Three launches on one workspace, then another batch shape and layout in the same bytes."""
     from ds355 import step
