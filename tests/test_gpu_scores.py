@@ -108,6 +108,47 @@ def test_head_reduce_max_matches_oracle(cuda, head_dim, chunk, block_size, dtype
     assert_scores_close(actual, expected)
 
 
+def _page_dense(dense, block_size, pad):
+    """Pages of the rows' dense keys [n, Hkv, D], in reverse order; rows of `pad` spare elements after each head."""
+    hkv, dim = dense[0].shape[1:]
+    pages = [(len(k) + block_size - 1) // block_size for k in dense]
+    store = torch.full((sum(pages), block_size, hkv, dim + pad), float("nan"), dtype=dense[0].dtype)[..., :dim]
+    table = torch.zeros((len(dense), max(pages)), dtype=torch.int32)
+    nxt = sum(pages)
+    for b, keys in enumerate(dense):
+        for p in range(pages[b]):
+            nxt -= 1
+            table[b, p] = nxt
+            part = keys[p * block_size:(p + 1) * block_size]
+            store[nxt, : len(part)] = part
+            store[nxt, len(part):] = 0.0
+    return store, table
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 192, 256])
+@pytest.mark.parametrize("block_size,pad", [(16, 0), (48, 8)])
+@pytest.mark.parametrize("mode", ["mean", "max", "free"])
+def test_whole_line_loads_give_the_bits_of_half_line_loads(cuda, head_dim, block_size, pad, mode):
+    # Blocks of whole 16-token groups read keys in 128-byte lines and exchange
+    # halves between lanes; other blocks (40 tokens) read the MFMA operands
+    # directly.  Same operands, same order: the same bits, at any row end
+    # within a group and with rows that are not line-aligned (pad).
+    g = gen(11)
+    lengths = [1, 7, 8, 9, 15, 16, 17, 63, 65, 500]
+    query = randn((len(lengths), 16, head_dim), torch.bfloat16, g)
+    dense = [randn((n, 2, head_dim), torch.bfloat16, g) for n in lengths]
+    lse = None if mode == "free" else torch.randn((len(lengths), 16), generator=g) + 4.0
+    out = []
+    for bs, extra in ((block_size, pad), (40, 0)):
+        keys, table = _page_dense(dense, bs, extra)
+        device_keys = torch.empty((*keys.shape[:3], head_dim + extra), dtype=keys.dtype, device=cuda)[..., :head_dim]
+        device_keys.copy_(keys)
+        out.append(_gpu_scores(query, device_keys, lse, table, lengths, 64, head_dim ** -0.5, cuda,
+                               head_reduce="max" if mode == "max" else "mean"))
+    assert torch.isfinite(out[0]).all()
+    assert torch.equal(out[0], out[1])
+
+
 def test_headline_shape_scores(cuda):
     """16 requests, L ~ U[4096, 40960], 32 q heads / 4 KV heads x 128, chunk 64."""
     g = gen(0)

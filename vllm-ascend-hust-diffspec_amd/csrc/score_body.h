@@ -117,6 +117,33 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(const Raw16& a, const Raw16& b, 
   }
 }
 
+// Keys in whole 128-byte lines.  The B operand wants 64 bytes of each of 16
+// tokens (lane kgrp * 16 + col: token col, 16-byte slice kgrp), so one load
+// per MFMA step reads half a line of every token, and a non-temporal load
+// then fetches each line twice.  Instead a pair of loads takes 128 bytes of
+// tokens 0-7 (lanes col < 8 slice kgrp, lanes col >= 8 slice 4 + kgrp of
+// token col - 8) and of tokens 8-15, and swap_lines exchanges the halves
+// between lanes col and col ^ 8: 12 VALU instructions per 2 KB, the operands
+// and so the results of the plain loads.  A bare read loop over 512 MB with
+// this address pattern: 5.8 TB/s cached, 6.65-6.8 non-temporal; the half-line
+// pattern 5.95 either way; contiguous 1 KB loads 6.0 and 6.8.  The steps with
+// it: 4 rows of 128k tokens 115.8 -> 100.2 us, 64 rows of 2-40k (64/8 heads)
+// 655 -> 606, 16 x 4-40k 97.8 -> 91.8, 16 x 8-40k without an LSE 119 -> 108;
+// 8 rows of 1-16k at head_dim 64 (49 MB of keys) 15.4 either way.
+__device__ __forceinline__ Raw16 load16_nt(const uint16_t* p) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(Raw16, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+}
+constexpr int kRowRor8 = 0x128;  // DPP: lane c of a 16-lane row reads lane c ^ 8
+__device__ __forceinline__ void swap_lines(Raw16& a, Raw16& b) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int x = static_cast<int>(a.w[w]), y = static_cast<int>(b.w[w]);
+    a.w[w] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(x, y, kRowRor8, 0xf, 0xc, false));
+    b.w[w] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(y, x, kRowRor8, 0xf, 0x3, false));
+  }
+}
+
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Raw buffer loads from a wave-uniform base (a resource in scalar registers)
@@ -251,6 +278,7 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
                                              const int* s_qrow, int total, int gw, int tw, uint32_t tag) {
   constexpr bool UNIFORM_PAGE = PAGE != PAGE_LANE;
   constexpr bool POW2 = PAGE == PAGE_POW2;
+  constexpr bool LINES = UNIFORM_PAGE && STEPS % 2 == 0;  // whole-line key loads (swap_lines)
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;   // A row (query head in group) / B column (token in group)
   const int kgrp = lane >> 4;  // 8-element k slice of the 32-wide MFMA step
@@ -351,7 +379,8 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
                           : 0;
   };
 
-  const int64_t lane_k = static_cast<int64_t>(col) * a.k_token_stride + kgrp * 8;
+  const int64_t lane_k = LINES ? static_cast<int64_t>(col & 7) * a.k_token_stride + kgrp * 8 + (col >> 3) * 32
+                               : static_cast<int64_t>(col) * a.k_token_stride + kgrp * 8;
   const int q_head = min(col, a.G - 1);  // rows >= G read a real head; masked later
 
   int last_qrow = -1, last_g = -1;  // (query row, KV head) of the last loaded batch (wave-uniform)
@@ -388,8 +417,17 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
                                : 0;
         krow = a.k + off + kgrp * 8;
       }
+      if constexpr (LINES) {
+        const uint16_t* krow8 = krow + 8 * a.k_token_stride;
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) out.k[i][s] = *reinterpret_cast<const Raw16*>(krow + 32 * s);
+        for (int s = 0; s < STEPS; s += 2) {
+          out.k[i][s] = load16_nt(krow + 32 * s);
+          out.k[i][s + 1] = load16_nt(krow8 + 32 * s);
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) out.k[i][s] = *reinterpret_cast<const Raw16*>(krow + 32 * s);
+      }
     }
   };
   // A batch of the same unit as the one just computed takes its q and LSE
@@ -437,7 +475,18 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
       const int ci = (tg * 16) >> a.ci_shift;
       f32x4_t logit = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s) logit = mfma16x16x32<DT>(bt.q[s], bt.k[i][s], logit);
+      for (int s = 0; s < STEPS; ++s) {
+        if constexpr (LINES) {
+          if (s % 2 == 0) {
+            Raw16 k0 = bt.k[i][s], k1 = bt.k[i][s + 1];
+            swap_lines(k0, k1);
+            logit = mfma16x16x32<DT>(bt.q[s], k0, logit);
+            logit = mfma16x16x32<DT>(bt.q[s + 1], k1, logit);
+          }
+        } else {
+          logit = mfma16x16x32<DT>(bt.q[s], bt.k[i][s], logit);
+        }
+      }
       const int tin = tg * 16 + col;
       const bool tok_ok = tin < a.U && c.t0 + tin < c.len;
       if (HMAX) {
