@@ -271,6 +271,19 @@ def test_random_rows_positions_and_groups(cuda, seed):
     _step(case, dev, cuda, slots, None, tokens, dim ** -0.5)
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("rows", [16, 320])
+def test_rows_that_end_inside_a_tile(cuda, dim, rows):
+    """Row ends at and beside the half tiles (8 tokens) that key loads take lines of, in the
+    one-shot kernel and (many rows) the streamed one."""
+    ends = [0, 1, 6, 7, 8, 9, 14, 15, 16, 17, 23, 24, 31, 32, 33, 63]
+    positions = (ends * (rows // 16))[:rows]
+    case = Case(17 + dim, rows, 4, 16, dim, 64)
+    for s, p in enumerate(positions):
+        case.fill(s, p)
+    _step(case, Device(case, cuda, rows), cuda, list(range(rows)), positions, rows, dim ** -0.5, device_positions=True)
+
+
 @pytest.mark.parametrize("rows,hq,hkv,dim,budget,dtype", [
     (20, 32, 4, 128, 2048, torch.bfloat16),  # 640 spans: just above one round of one-shot workgroups
     (33, 8, 8, 64, 2304, torch.float16),  # one query head per KV head

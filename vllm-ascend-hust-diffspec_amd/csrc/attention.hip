@@ -24,12 +24,11 @@
 //                                     index lane / 16 is token 4 * (lane / 16)
 //                                     + i, so the B operand is the lane's own
 //                                     probability; head_dim column m of block
-//                                     j is d = J * m + j (J = D / 16), so the
-//                                     A operand is one contiguous J-element
-//                                     vector of V's row, and each lane ends
-//                                     with the D / 4 contiguous outputs
-//                                     [4J * (lane / 16), 4J * (lane / 16 + 1))
-//                                     of query g.
+//                                     j is d = out_dim(m, j) (J = D / 16
+//                                     blocks), so the A operand is the
+//                                     elements of V's row that lane column m
+//                                     loads, and each lane ends with D / 4
+//                                     outputs of query g.
 // Probabilities stay fp32 (the reference's softmax is fp32 and multiplies
 // fp32 V).  The four waves merge in LDS.  A row that fits one span writes its
 // output directly; in a longer row every span but the last writes its
@@ -136,6 +135,29 @@ __device__ __forceinline__ float unpack(uint32_t w, int half) {
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
+// Working rows are read in whole 128-byte lines, non-temporally (a bare read
+// loop on this card: 5.95 TB/s cached or in half lines, 6.7-6.9 TB/s so).  The
+// A operand of the score MFMAs wants 64 bytes of each of 16 tokens (lane quad
+// * 16 + col: token col, 16-byte slice quad).  Loads 2 p and 2 p + 1 of a tile
+// therefore take line p of tokens 0-7 and of tokens 8-15: lane (quad, col)
+// holds slice quad + 4 (col / 8) of token (col % 8) + 8 (i % 2), and
+// swap_lines exchanges halves between lanes col and col ^ 8.
+constexpr int kPolicyNt = 2;
+__device__ __forceinline__ u32x4 load16_nt(const uint16_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+__device__ __forceinline__ int line_token(int col, int i) { return (col & 7) + 8 * (i & 1); }
+__device__ __forceinline__ int line_elem(int quad, int col, int i) { return 8 * quad + 32 * (col >> 3) + 64 * (i >> 1); }
+constexpr int kRowRor8 = 0x128;  // DPP: lane c of a 16-lane row reads lane c ^ 8
+__device__ __forceinline__ void swap_lines(u32x4& a, u32x4& b) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int x = static_cast<int>(a[w]), y = static_cast<int>(b[w]);
+    a[w] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(x, y, kRowRor8, 0xf, 0xc, false));
+    b[w] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(y, x, kRowRor8, 0xf, 0x3, false));
+  }
+}
+
 // p = hi + lo in the cache dtype (16-bit words).  bf16: hi is p cut to its
 // top 16 bits (exact), lo the remainder p - hi (exact in fp32) cut the same
 // way, so |p - hi - lo| < 2^-14 |p|.  fp16: hi is p rounded to fp16, lo the
@@ -154,16 +176,24 @@ __device__ __forceinline__ void split_prob(float p, uint32_t& hi, uint32_t& lo) 
   }
 }
 
-// J consecutive 16-bit elements (J = 4, 8 or 16) as J / 2 words.
+// The J = D / 16 elements of a V row that lane column m reads, as J / 2 words:
+// J m .. J m + J - 1 for J <= 8 (16 lanes cover the row); for J = 16 8 m .. 8 m
+// + 7 of each half of the row, so that either load of 16 lanes covers whole
+// lines.  out_dim is the head_dim index of element j.
 template <int J>
+__device__ __forceinline__ constexpr int v_elem(int m) { return (J < 8 ? J : 8) * m; }
+template <int J>
+__device__ __forceinline__ constexpr int out_dim(int m, int j) { return v_elem<J>(m) + (j & 7) + (j >> 3) * 128; }
+template <int J, bool NT>
 __device__ __forceinline__ void load_words(const uint16_t* p, uint32_t (&w)[J / 2]) {
   if constexpr (J == 4) {
-    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+    const u32x2 v = NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p))
+                       : *reinterpret_cast<const u32x2*>(p);
     w[0] = v.x; w[1] = v.y;
   } else {
 #pragma unroll
     for (int h = 0; h < J / 8; ++h) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(p + 8 * h);
+      const u32x4 v = NT ? load16_nt(p + 128 * h) : load16(p + 128 * h);
       w[4 * h] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
     }
   }
@@ -189,16 +219,16 @@ __device__ __forceinline__ f32x2 load8_sc1(Rsrc16 r, uint32_t off) {
   return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(off), 0, kPolicySc1));
 }
 
-// J consecutive 16-bit elements through a buffer resource.
+// The same through a buffer resource, non-temporally.
 template <int J>
 __device__ __forceinline__ void load_words_buf(Rsrc16 r, int voff, int soff, uint32_t (&w)[J / 2]) {
   if constexpr (J == 4) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kPolicyNt);
     w[0] = v.x; w[1] = v.y;
   } else {
 #pragma unroll
     for (int h = 0; h < J / 8; ++h) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * h, soff, 0);
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 256 * h, soff, kPolicyNt);
       w[4 * h] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
     }
   }
@@ -275,9 +305,14 @@ __device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv
   sc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
   sc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < AttnShape<D>::kSteps; ++i) {
-    sc[0] = mfma_scores<DT>(T.k[0][i], qv[i], sc[0]);
-    sc[1] = mfma_scores<DT>(T.k[1][i], qv[i], sc[1]);
+  for (int i = 0; i < AttnShape<D>::kSteps; i += 2) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4 k0 = T.k[h][i], k1 = T.k[h][i + 1];
+      swap_lines(k0, k1);
+      sc[h] = mfma_scores<DT>(k0, qv[i], sc[h]);
+      sc[h] = mfma_scores<DT>(k1, qv[i + 1], sc[h]);
+    }
   }
 }
 
@@ -285,7 +320,7 @@ __device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv
 // all).  The output MFMAs are 16x16x32 in the cache dtype with A = V^T and
 // B = P^T: k-slot (lane / 16, e) is token 4 * (lane / 16) + (e & 3) of tile
 // e / 4, i.e. the rows of the lane's own score tiles, and head_dim column m of
-// block j is d = J * m + j, so both operands are in the lane's registers.  P
+// block j is out_dim(m, j), so both operands are in the lane's registers.  P
 // is split into an upper part (its fp32 value cut to the dtype) and the dtype
 // rounding of the exact remainder; two MFMAs per block keep the products
 // within ~2^-16 of fp32 probabilities.
@@ -350,7 +385,6 @@ __device__ __forceinline__ void waves_to_lds(MergeShared<D>& sh, const Running<D
   float l = run.l;
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  const int d0 = 4 * J * quad;  // lane's outputs: d = d0 + J * i + j
   if (quad == 0) {
     sh.m[wave][col] = run.m;
     sh.l[wave][col] = l;
@@ -358,7 +392,7 @@ __device__ __forceinline__ void waves_to_lds(MergeShared<D>& sh, const Running<D
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int j = 0; j < J; ++j) sh.acc[wave][col][d0 + J * i + j] = run.acc[j][i];
+    for (int j = 0; j < J; ++j) sh.acc[wave][col][out_dim<J>(4 * quad + i, j)] = run.acc[j][i];
   }
 }
 
@@ -577,13 +611,15 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   auto load_rows = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint16_t* pk = kw + static_cast<int64_t>(min(tb + h * kTileT + col, a.budget - 1)) * D + 8 * quad;
 #pragma unroll
-      for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = load16(pk + 32 * i);
+      for (int i = 0; i < S::kSteps; ++i) {
+        const int t = min(tb + h * kTileT + line_token(col, i), a.budget - 1);
+        K.k[h][i] = load16_nt(kw + static_cast<int64_t>(t) * D + line_elem(quad, col, i));
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        load_words<J>(vw + static_cast<int64_t>(min(tb + h * kTileT + 4 * quad + r, a.budget - 1)) * D + J * col,
-                      V.v[h][r]);
+        const int t = min(tb + h * kTileT + 4 * quad + r, a.budget - 1);
+        load_words<J, true>(vw + static_cast<int64_t>(t) * D + v_elem<J>(col), V.v[h][r]);
       }
     }
   };
@@ -593,14 +629,14 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   // position: working rows below the cache capacity and the input row.
   KTiles<D> k0, k1;
   VTiles<D> v0, v1;
-  u32x4 kin_s[S::kSteps];
+  u32x4 kin_s[S::kSteps / 2];  // the lane's slice of each line
   uint32_t vin_s[J / 2];
   const bool early = real && slot_ok && t0 < a.budget;
   if (early) {
     load_rows(k0, v0, t0);
 #pragma unroll
-    for (int i = 0; i < S::kSteps; ++i) kin_s[i] = load16(kin + 8 * quad + 32 * i);
-    load_words<J>(vin + J * col, vin_s);
+    for (int i = 0; i < S::kSteps; i += 2) kin_s[i / 2] = load16(kin + line_elem(quad, col, i));
+    load_words<J, false>(vin + v_elem<J>(col), vin_s);
   }
   lds_barrier();
   const int pos = s_pos;
@@ -655,11 +691,14 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   auto load_pair = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint16_t* pk = row_ptr(kw, kin, tb + h * kTileT + col) + 8 * quad;
 #pragma unroll
-      for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = load16(pk + 32 * i);
+      for (int i = 0; i < S::kSteps; ++i) {
+        K.k[h][i] = load16_nt(row_ptr(kw, kin, tb + h * kTileT + line_token(col, i)) + line_elem(quad, col, i));
+      }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) load_words<J>(row_ptr(vw, vin, tb + h * kTileT + 4 * quad + r) + J * col, V.v[h][r]);
+      for (int r = 0; r < 4; ++r) {
+        load_words<J, true>(row_ptr(vw, vin, tb + h * kTileT + 4 * quad + r) + v_elem<J>(col), V.v[h][r]);
+      }
     }
   };
   // A pair loaded from the working rows: the position's row becomes the
@@ -669,9 +708,9 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   auto fix_pair = [&](KTiles<D>& K, VTiles<D>& V, int tb) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (tb + h * kTileT + col == pos) {
 #pragma unroll
-        for (int i = 0; i < S::kSteps; ++i) K.k[h][i] = kin_s[i];
+      for (int i = 0; i < S::kSteps; ++i) {
+        if (tb + h * kTileT + line_token(col, i) == pos) K.k[h][i] = kin_s[i / 2];
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -746,14 +785,14 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
 // start, and 4 waves x 16 KB in flight per CU already fill the memory queue.
 // us on 57 rows of 300-3970 tokens (64/8 heads x 128, fp16) / 64 rows of 1987
 // (32/4 x 128) / 16 rows of 1984-3990 (32/8 x 256) / 48 rows of 984-1990
-// (32/8 x 64); bandwidth of the last line 5.0, 5.5, 5.0 and 4.4 TB/s:
-//   one workgroup per span                          184 / 63 / 130 / 43.5
-//   ranges, 3 workgroups per CU (2 at 256, 4 at 64) 118 / 64 / 121 / 38.0
-//   ranges, 2 (2, 3)                                106 / 52 / 121 / 37.6
-//   ranges, 1 (1, 2), kept                          107 / 48 /  82 / 34.8
-// (at 256 two per CU spill 42 registers).  Two steps in flight per wave: 110
-// / 48.6 / 82 / 35.5.  The next unit's operands requested before the merge:
-// 105 / 54 / 82 / 34.9, no gain for 35 more registers.
+// (32/8 x 64); bandwidth of the last line 5.5, 6.1, 5.6 and 4.9 TB/s:
+//   one workgroup per span, cached half lines       184 / 63 / 130 / 43.5
+//   ranges, 1 workgroup per CU (2 at 64), the same  107 / 48 /  82 / 34.8
+//   whole lines, non-temporal, 2 (2, 3) per CU       94 / 46.5 / 71 / 32.8
+//   whole lines, non-temporal, 1 (1, 2) per CU, kept 98 / 42.8 / 70 / 30.2
+// With the cached reads: two steps in flight per wave 110 / 48.6 / 82 / 35.5;
+// the next unit's operands requested before the merge 105 / 54 / 82 / 34.9,
+// no gain for 35 more registers.
 template <int D>
 struct StreamShape {
   static constexpr int kStep = kWavesA * 2 * kTileT;            // tokens per step (32 per wave)
@@ -865,8 +904,8 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
   // rows (a scalar base, one lane offset, fixed steps).  Rows at or past the
   // position come from the new token's input row instead (its scores past
   // the position are masked): the unit's last waves choose per lane.
-  const int k_lane = (col * D + 8 * quad) * 2;
-  const int v_lane = (4 * quad * D + J * col) * 2;
+  const int k_lane = (line_token(col, 0) * D + line_elem(quad, col, 0)) * 2;
+  const int v_lane = (4 * quad * D + v_elem<J>(col)) * 2;
   const int unit_bytes = a.budget * D * 2;
   auto load_k = [&](KTiles<D>& T, const Unit& u, int token) {
     const int tb = __builtin_amdgcn_readfirstlane(token);
@@ -878,17 +917,19 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
         const int at = (tb + h * kTileT) * D * 2;
 #pragma unroll
         for (int i = 0; i < S::kSteps; ++i) {
-          T.k[h][i] = __builtin_amdgcn_raw_buffer_load_b128(r, k_lane + 64 * i, at, 0);
+          T.k[h][i] = __builtin_amdgcn_raw_buffer_load_b128(r, k_lane + 16 * (i & 1) * D + 128 * (i >> 1), at,
+                                                            kPolicyNt);
         }
       }
     } else {
       const uint16_t* in = kin_of(u);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int t = tb + h * kTileT + col;
-        const uint16_t* p = (t >= u.pos ? in : rows_k + static_cast<int64_t>(t) * D) + 8 * quad;
 #pragma unroll
-        for (int i = 0; i < S::kSteps; ++i) T.k[h][i] = load16(p + 32 * i);
+        for (int i = 0; i < S::kSteps; ++i) {
+          const int t = tb + h * kTileT + line_token(col, i);
+          T.k[h][i] = load16((t >= u.pos ? in : rows_k + static_cast<int64_t>(t) * D) + line_elem(quad, col, i));
+        }
       }
     }
   };
@@ -909,7 +950,7 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int t = tb + h * kTileT + 4 * quad + r;
-          load_words<J>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + J * col, T.v[h][r]);
+          load_words<J, false>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + v_elem<J>(col), T.v[h][r]);
         }
       }
     }
