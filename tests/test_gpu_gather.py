@@ -116,6 +116,38 @@ def test_gather_dtypes_and_layouts(cuda, dtype, neox, rotary_dim):
     assert torch.equal(torch.nan_to_num(got_k), torch.nan_to_num(exp_k))
 
 
+@pytest.mark.parametrize("dtype,dim,rotary_dim,neox", [
+    (torch.bfloat16, 64, 64, True), (torch.bfloat16, 64, 32, True), (torch.float16, 64, 32, False),
+    (torch.float16, 64, 64, True), (torch.float32, 32, 16, False), (torch.float32, 32, 32, True)])
+@pytest.mark.parametrize("heads", [1, 5, 8])
+def test_gather_rows_of_one_line(cuda, dtype, dim, rotary_dim, neox, heads):
+    """Rows of 128 bytes, moved in whole lines by pairs of lanes: histories that end inside and
+    beside a task's 16 positions, heads in one and several groups."""
+    chunk, token_budget, lmax = 32, 512, 900
+    g = gen(9)
+    ends = [1, 2, 3, 4, 7, 15, 16, 17, 18, 31, 33, 480, 899]
+    slots = list(reversed(range(len(ends))))
+    budget = O.history_budget(token_budget, 4, chunk)
+    plans = []
+    for slot, end in zip(slots, ends):
+        scores = torch.rand((end + chunk) // chunk, generator=g)
+        sel = O.select_context_chunks(scores, end + 1, chunk, budget)
+        plans.append(O.history_plan(slot, sel.chunk_indices.tolist(), end, chunk, budget))
+    plan = O.pad_plan(plans, token_budget, chunk)
+    raw_k = randn((len(ends), lmax, heads, dim), dtype, g)
+    raw_v = randn((len(ends), lmax, heads, dim), dtype, g)
+    cos_sin = O.rope_cos_sin_cache(rotary_dim, token_budget, dtype=dtype)
+    exp_k = torch.full((len(ends), heads, token_budget, dim), float("nan"), dtype=dtype)
+    exp_v = exp_k.clone()
+    O.rebuild_compact_kv_from_plan(raw_k, raw_v, exp_k, exp_v, plan, cos_sin, chunk_size=chunk,
+                                   max_width=budget, rotary_dim=rotary_dim, is_neox_style=neox)
+    work_k, work_v = torch.full_like(exp_k, float("nan")).to(cuda), torch.full_like(exp_v, float("nan")).to(cuda)
+    _run_batched(raw_k.to(cuda), raw_v.to(cuda), work_k, work_v, plan, cos_sin, chunk, budget, rotary_dim, neox, cuda)
+    for got, exp in ((work_k.cpu(), exp_k), (work_v.cpu(), exp_v)):
+        assert torch.equal(got.isnan(), exp.isnan())
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(exp))
+
+
 def test_gather_scalar_fallback_matches_oracle(cuda):
     """Shapes the 16-byte path does not cover (head_dim 6, rotary 2..6) take the element path."""
     g = gen(9)

@@ -534,12 +534,12 @@ __device__ __forceinline__ bool poll_plan(const FusedArgs& f, int r, uint32_t ta
 }
 
 // Gather task t (local positions t * ppw ...) of the row in `v`.
-template <int DT, bool NEOX>
+template <int DT, bool NEOX, bool LINES>
 __device__ __forceinline__ void run_task(const gather::GatherArgs& ga, const gather::GatherLane& L,
                                          const PlanView& v, int t) {
   const int ppw = 64 / ga.lanes_per_row;
-  gather::gather_task<DT, NEOX, kGatherHeads>(
-      ga, L, t * ppw, v.slot, v.len, v.tail_start, v.prefix_len, v.drop, [&](int64_t c) {
+  gather::gather_task<DT, NEOX, kGatherHeads, gather::kLoadNT, LINES>(
+      ga, L, t * ppw, v.slot, v.len, v.tail_start, v.prefix_len, v.drop, 0, ga.heads, [&](int64_t c) {
         // Chunk id column 5 + c sits in lane (5 + c) % 64 of lo or hi.
         const int col = static_cast<int>(5 + c);
         const int lo = __builtin_amdgcn_ds_bpermute((col & 63) << 2, static_cast<int>(v.lo));
@@ -558,7 +558,7 @@ __device__ __forceinline__ uint64_t task_record(const FusedArgs& f, int slot, in
 // Gather task t of the row in `v`, keeping its gather record: a task whose
 // record shows the working cache already holds its bytes is left out, and
 // with prefix_only so is every task not wholly in the history prefix.
-template <int DT, bool NEOX>
+template <int DT, bool NEOX, bool LINES>
 __device__ __forceinline__ void gather_recorded(const FusedArgs& f, const gather::GatherLane& L, const PlanView& v,
                                                 int r, int t, uint64_t have) {
   const int ppw = 64 / f.g.lanes_per_row;
@@ -577,7 +577,7 @@ __device__ __forceinline__ void gather_recorded(const FusedArgs& f, const gather
     if (want != 0u && have == want) move = false;
     if ((threadIdx.x & 63) == 0 && have != want) f.rec[v.slot * f.rec_stride + t] = want;
   }
-  if (move) run_task<DT, NEOX>(f.g, L, v, t);
+  if (move) run_task<DT, NEOX, LINES>(f.g, L, v, t);
 }
 
 // A scoring wave's gather tasks: task numbers gw, gw + tw, ... of the
@@ -587,7 +587,7 @@ __device__ __forceinline__ void gather_recorded(const FusedArgs& f, const gather
 // word is set, for the last workgroup to finish.  Both writes are
 // read-modify-writes the wave waits for, so they are in memory before its
 // workgroup counts itself done.
-template <int DT, bool NEOX>
+template <int DT, bool NEOX, bool LINES>
 __device__ __forceinline__ void gather_owned(const FusedArgs& f, const int* task_prefix, const int* row_slot, int gw,
                                              int tw, uint32_t tag) {
   const gather::GatherArgs& ga = f.g;
@@ -612,7 +612,7 @@ __device__ __forceinline__ void gather_owned(const FusedArgs& f, const int* task
       published = poll_plan(f, r, tag, f.owner_spins, v);
     }
     if (published) {
-      gather_recorded<DT, NEOX>(f, L, v, r, t, have);
+      gather_recorded<DT, NEOX, LINES>(f, L, v, r, t, have);
     } else if ((threadIdx.x & 63) == 0) {
       __hip_atomic_exchange(f.state + static_cast<int64_t>(r) * f.task_cap + t, tag | kSkipped, __ATOMIC_ACQUIRE,
                             __HIP_MEMORY_SCOPE_AGENT);
@@ -626,7 +626,7 @@ __device__ __forceinline__ void gather_owned(const FusedArgs& f, const int* task
 // published and every skip mark is in memory.  Each wave checks 64 tasks of
 // a row at a time.  A bit a wait raises here goes straight to the owner's
 // words, since the launch's status word has already been handed over.
-template <int DT, bool NEOX>
+template <int DT, bool NEOX, bool LINES>
 __device__ __forceinline__ void redo_skipped(const FusedArgs& f, const int* task_prefix, uint32_t tag) {
   const int lane = threadIdx.x & 63;
   const gather::GatherLane L = gather::gather_lane<DT, NEOX>(f.g);
@@ -655,7 +655,7 @@ __device__ __forceinline__ void redo_skipped(const FusedArgs& f, const int* task
             break;
           }
         }
-        gather_recorded<DT, NEOX>(f, L, v, b, t0 + k, task_record(f, static_cast<int>(v.slot), t0 + k));
+        gather_recorded<DT, NEOX, LINES>(f, L, v, b, t0 + k, task_record(f, static_cast<int>(v.slot), t0 + k));
       }
     }
   }
@@ -670,6 +670,10 @@ struct WorkShared {
 
 template <int DT, int STEPS, bool NEOX, int PAGE, bool LSEFREE>
 __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
+  // Whole-line gathers where the target's head_dim, and so usually the
+  // draft's, is 64 (the code for them costs 1.7 us of 108 on 16 rows without
+  // an LSE at head_dim 128, which never runs it).
+  constexpr bool LINES = STEPS == 2;
   constexpr int KB = STEPS <= 2 ? 2 : 1;  // chunk_score_kernel's batch shape (4 KB) for head_dim <= 128
   __shared__ union {
     select::SelectShared<kFusedKeys> sel;
@@ -744,7 +748,7 @@ __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
     const int tw = first_selector * kWaves;
     score::score_stream<DT, STEPS, KB, false, PAGE, true, LSEFREE>(sa, w.unit_prefix, w.len, w.qrow,
                                                                    w.unit_prefix[rows], gw, tw, tag);
-    gather_owned<DT, NEOX>(f, s_task_prefix, s_slot, gw, tw, tag);
+    gather_owned<DT, NEOX, LINES>(f, s_task_prefix, s_slot, gw, tw, tag);
   }
 
   // The last workgroup to finish hands this launch's status bits to the
@@ -778,7 +782,7 @@ __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
   }
   __syncthreads();
   if (s_last == 3u) {
-    redo_skipped<DT, NEOX>(f, s_task_prefix, tag);
+    redo_skipped<DT, NEOX, LINES>(f, s_task_prefix, tag);
     if (threadIdx.x == 0) {
       coherent_store(f.header + kDone, 0u);
       coherent_store(f.header + kEpoch, tag);

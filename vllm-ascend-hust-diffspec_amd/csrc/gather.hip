@@ -20,8 +20,8 @@ namespace {
 using namespace gather;
 
 // Vectorised path.  Waves are independent workers (no block barrier after
-// the prologue).  A task is (row, ppw consecutive local positions) for every
-// head; ppw = 64 / lanes_per_row.  Lane l owns position p0 + l / lanes_per_row
+// the prologue).  A task is (row, ppw consecutive local positions, HG
+// heads); ppw = 64 / lanes_per_row.  Lane l owns position p0 + l / lanes_per_row
 // and slice j = l % lanes_per_row of the head dimension, where it moves two
 // 16-byte K vectors and two 16-byte V vectors per head:
 //   neox : slices [0, half/V) rotate the pair (jV, half + jV); the other
@@ -29,12 +29,13 @@ using namespace gather;
 //   gptj : slice j handles vectors jV and D/2 + jV, each rotated in place
 //          when below rot, copied otherwise.
 //   V    : slice j copies vectors jV and D/2 + jV.
-// The cos/sin vectors of the lane's position are loaded once and reused for
-// every head.  Plan fields are wave-uniform and come through scalar loads;
+// A task covers HG heads, whose loads are all in flight at once (in a loop over
+// more heads, the next round's data waits for this round's stores).  The
+// cos/sin vectors of the lane's position are loaded once for them.  Plan fields are wave-uniform and come through scalar loads;
 // only the chunk id of a prefix position is a per-lane load.  Resources span
 // one slot's raw cache ([max_model_len, H, D], below 2 GiB: checked on the
 // host) and one slot's working cache ([H, budget, D]); a lane with nothing
-// to move uses an out-of-range offset.  HG = heads in flight at once.
+// to move uses an out-of-range offset.
 template <int DT, bool NEOX, int HG>
 __global__ __launch_bounds__(kThreads) void gather_wave_kernel(GatherArgs a) {
   __shared__ int s_prefix[kMaxRows + 1];
@@ -42,13 +43,16 @@ __global__ __launch_bounds__(kThreads) void gather_wave_kernel(GatherArgs a) {
 
   const int ppw = 64 / a.lanes_per_row;
   build_row_prefix(a.rows, s_prefix, s_scratch, [&](int r) { return (row_len(a, r) + ppw - 1) / ppw; });
-  const int total = s_prefix[a.rows];
+  const int groups = (a.heads + HG - 1) / HG;
+  const int total = s_prefix[a.rows] * groups;
   const GatherLane L = gather_lane<DT, NEOX>(a);
 
   const int gw = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
   const int tw = gridDim.x * (kThreads / 64);
   int hint = 0;
-  for (int task = gw; task < total; task += tw) {
+  for (int item = gw; item < total; item += tw) {
+    const int task = groups == 1 ? item : item / groups;
+    const int h0 = (item - task * groups) * HG;
     int lo = hint, hi = a.rows - 1;  // task numbers grow along the wave's list
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
@@ -63,7 +67,7 @@ __global__ __launch_bounds__(kThreads) void gather_wave_kernel(GatherArgs a) {
     const int64_t tail_start = scalar_load(prow + 2);
     const int64_t prefix_len = scalar_load(prow + 3);
     const int64_t drop = scalar_load(prow + 4);
-    gather_task<DT, NEOX, HG>(a, L, p0, slot, len, tail_start, prefix_len, drop,
+    gather_task<DT, NEOX, HG, kLoadCached, true>(a, L, p0, slot, len, tail_start, prefix_len, drop, h0, min(h0 + HG, a.heads),
                               [&](int64_t c) { return prow[5 + c]; });
   }
 }
@@ -240,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void plan_gather_kernel(GatherArgs a, Pla
   }
   if (!move) return;
   const GatherLane L = gather_lane<DT, NEOX>(a);
-  gather_task<DT, NEOX, HG>(a, L, p0, slot, limit, tail_start, prefix_len, drop, [&](int64_t c) {
+  gather_task<DT, NEOX, HG, kLoadCached, true>(a, L, p0, slot, limit, tail_start, prefix_len, drop, 0, a.heads, [&](int64_t c) {
     const int col = static_cast<int>(c);
     const int l = __builtin_amdgcn_ds_bpermute((col & 63) << 2, static_cast<int>(lo));
     const int h = __builtin_amdgcn_ds_bpermute((col & 63) << 2, static_cast<int>(hi));
@@ -311,7 +315,8 @@ template <int DT>
 int launch_gather(hipStream_t stream, const GatherArgs& a, bool neox, bool vec, int grid) {
   if (vec) {
     const int ppw = 64 / a.lanes_per_row;
-    const int64_t tasks = static_cast<int64_t>(a.rows) * ((a.pos_limit + ppw - 1) / ppw);
+    const int hg = a.heads >= 4 ? 4 : (a.heads >= 2 ? 2 : 1);
+    const int64_t tasks = static_cast<int64_t>(a.rows) * ((a.pos_limit + ppw - 1) / ppw) * ((a.heads + hg - 1) / hg);
     if (a.heads >= 4) {
       if (neox) return launch_wave<gather_wave_kernel<DT, true, 4>>(stream, a, tasks);
       return launch_wave<gather_wave_kernel<DT, false, 4>>(stream, a, tasks);

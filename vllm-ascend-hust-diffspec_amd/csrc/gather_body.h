@@ -150,8 +150,9 @@ constexpr uint32_t kOutOfRange = 0x80000000u;  // beyond every resource size use
 __device__ __forceinline__ Rsrc make_rsrc(const void* base, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
 }
+template <int POLICY = 0>
 __device__ __forceinline__ W4 buf_load16(Rsrc r, uint32_t voff, uint32_t soff) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(voff), static_cast<int>(soff), 0);
+  return __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(voff), static_cast<int>(soff), POLICY);
 }
 __device__ __forceinline__ W2 buf_load8(Rsrc r, uint32_t voff) {
   return __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(voff), 0, 0);
@@ -161,8 +162,41 @@ __device__ __forceinline__ W2 buf_load8(Rsrc r, uint32_t voff) {
 // displacing cached lines, measured about 15% faster than cached stores when
 // the gathered rows are not already in the MALL.
 constexpr int kStoreNT = 2;
+// Policy of the raw rows' loads.  The single launch, where the scored keys
+// stream past, reads them non-temporally (16 rows of 4-40k: 92.2 -> 89.0 us);
+// the gather kernels read them cached (non-temporal: 24 rows at head_dim 64
+// 34.6 -> 36.4 us, one 8k row 17.7 -> 18.4, 4 rows of 128k 100.3 -> 101.3).
+constexpr int kLoadCached = 0;
+constexpr int kLoadNT = 2;
 __device__ __forceinline__ void buf_store16(W4 v, Rsrc r, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_buffer_store_b128(v, r, static_cast<int>(voff), static_cast<int>(soff), kStoreNT);
+}
+
+// Rows of 128 bytes (head_dim 64 in 16 bits, 32 in 32) in whole lines.  A
+// lane's two vectors of a position lie in two loads, so 4 lanes a row would
+// read and write half lines, the second half with another instruction; a
+// non-temporal half line moves whole to and from memory.  Instead lanes l and
+// l ^ 8 (positions q and q ^ 2) share the work of both positions: the lane
+// with bit 3 clear takes the first vector of each, the other the second, and
+// the swap brings the two vectors of its own position to each lane where a
+// rotation needs both (and back for the stores).  24 rows of 130-9001 tokens
+// (8 heads x 64, fp16): 39.9 -> 34.6 us together with one round of heads per
+// task (gather_wave_kernel).
+constexpr int kRowRor8 = 0x128;  // DPP: lane c of a 16-lane row reads lane c ^ 8
+__device__ __forceinline__ uint32_t from_lane8(uint32_t own, uint32_t other, int keep_low) {
+  // Lanes with bit 3 set (keep_low) or clear get `other` of lane ^ 8; the rest keep `own`.
+  return static_cast<uint32_t>(keep_low ? __builtin_amdgcn_update_dpp(static_cast<int>(own), static_cast<int>(other),
+                                                                      kRowRor8, 0xf, 0xc, false)
+                                        : __builtin_amdgcn_update_dpp(static_cast<int>(own), static_cast<int>(other),
+                                                                      kRowRor8, 0xf, 0x3, false));
+}
+__device__ __forceinline__ void swap_lines(W4& a, W4& b) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const uint32_t x = a[w], y = b[w];
+    a[w] = from_lane8(x, y, 1);
+    b[w] = from_lane8(y, x, 0);
+  }
 }
 
 // Per-lane constants of the vector path, computed once per wave.
@@ -178,6 +212,7 @@ struct GatherLane {
   uint32_t raw_head, work_head;
   Rsrc cs;
   int ncol;  // chunk-id columns of a plan row
+  bool lines;  // rows of 128 bytes: whole-line accesses (swap_lines)
 };
 
 template <int DT, bool NEOX>
@@ -226,16 +261,18 @@ __device__ __forceinline__ GatherLane gather_lane(const GatherArgs& a) {
   L.work_head = static_cast<uint32_t>(static_cast<int64_t>(a.budget) * D * SZ);
   L.cs = make_rsrc(a.cos_sin, static_cast<int64_t>(a.pos_limit) * a.cs_stride * SZ);
   L.ncol = a.plan_width - 5;
+  L.lines = lpr == 4;
   return L;
 }
 
 // Moves local positions p0 .. p0 + ppw - 1 of one plan row (fields slot ..
 // drop, wave-uniform; len already clamped to pos_limit and 0 for an invalid
-// slot).  chunk_id(c) returns the plan row's chunk id column c.
-template <int DT, bool NEOX, int HG, typename ChunkId>
+// slot), heads h_begin .. h_end - 1.  chunk_id(c) returns the plan row's chunk
+// id column c.  LINES: rows of one line are moved in whole lines.
+template <int DT, bool NEOX, int HG, int POLICY, bool LINES, typename ChunkId>
 __device__ __forceinline__ void gather_task(const GatherArgs& a, const GatherLane& L, int p0, int64_t slot,
                                             int64_t len, int64_t tail_start, int64_t prefix_len, int64_t drop,
-                                            ChunkId chunk_id) {
+                                            int h_begin, int h_end, ChunkId chunk_id) {
   using T = typename Elem<DT>::T;
   constexpr int V = 16 / sizeof(T);
   constexpr int SZ = sizeof(T);
@@ -269,6 +306,21 @@ __device__ __forceinline__ void gather_task(const GatherArgs& a, const GatherLan
   const uint32_t src = ok ? static_cast<uint32_t>(pos * H * D * SZ) : kOutOfRange;
   const uint32_t dst = ok ? static_cast<uint32_t>(p * D * SZ) : kOutOfRange;
   const uint32_t csr = ok ? static_cast<uint32_t>(p * a.cs_stride * SZ) : kOutOfRange;
+  // Byte offsets of the lane's two vectors: its own position's, or with whole
+  // lines its half of positions q & ~2 and q | 2 (out of range where that
+  // position moves nothing).
+  const bool lines = LINES && L.lines;
+  uint32_t src0 = src, src1 = src, dst0 = dst, dst1 = dst;
+  int ko0 = k_off0 * SZ, ko1 = k_off1 * SZ, vo0 = v_off0 * SZ, vo1 = v_off1 * SZ;
+  if (lines) {  // wave-uniform
+    src0 = from_lane8(src, src, 1);
+    src1 = from_lane8(src, src, 0);
+    dst0 = from_lane8(dst, dst, 1);
+    dst1 = from_lane8(dst, dst, 0);
+    const bool second = (q & 2) != 0;
+    ko0 = ko1 = second ? ko1 : ko0;
+    vo0 = vo1 = second ? vo1 : vo0;
+  }
 
   W4 c16 = W4{0u, 0u, 0u, 0u}, s16 = W4{0u, 0u, 0u, 0u};
   W2 c8a = W2{0u, 0u}, s8a = W2{0u, 0u}, c8b = W2{0u, 0u}, s8b = W2{0u, 0u};
@@ -288,19 +340,20 @@ __device__ __forceinline__ void gather_task(const GatherArgs& a, const GatherLan
     }
   }
 
-  for (int h0 = 0; h0 < H; h0 += HG) {
+  for (int h0 = h_begin; h0 < h_end; h0 += HG) {
     W4 k0[HG], k1[HG], v0[HG], v1[HG];
 #pragma unroll
     for (int u = 0; u < HG; ++u) {
-      const uint32_t hs = static_cast<uint32_t>(min(h0 + u, H - 1)) * raw_head;
-      k0[u] = buf_load16(rk, src + k_off0 * SZ, hs);
-      k1[u] = buf_load16(rk, src + k_off1 * SZ, hs);
-      v0[u] = buf_load16(rv, src + v_off0 * SZ, hs);
-      v1[u] = buf_load16(rv, src + v_off1 * SZ, hs);
+      const uint32_t hs = static_cast<uint32_t>(min(h0 + u, h_end - 1)) * raw_head;
+      k0[u] = buf_load16<POLICY>(rk, src0 + ko0, hs);
+      k1[u] = buf_load16<POLICY>(rk, src1 + ko1, hs);
+      v0[u] = buf_load16<POLICY>(rv, src0 + vo0, hs);
+      v1[u] = buf_load16<POLICY>(rv, src1 + vo1, hs);
     }
 #pragma unroll
     for (int u = 0; u < HG; ++u) {
-      if (h0 + u >= H) break;  // wave-uniform
+      if (h0 + u >= h_end) break;  // wave-uniform
+      if (lines) swap_lines(k0[u], k1[u]);
       W4 ok0 = k0[u], ok1 = k1[u];
       if constexpr (DT == DS_BF16) {
         if (NEOX) {
@@ -370,10 +423,11 @@ __device__ __forceinline__ void gather_task(const GatherArgs& a, const GatherLan
         }
       }
       const uint32_t hd = static_cast<uint32_t>(h0 + u) * work_head;
-      buf_store16(ok0, wk, dst + k_off0 * SZ, hd);
-      buf_store16(ok1, wk, dst + k_off1 * SZ, hd);
-      buf_store16(v0[u], wv, dst + v_off0 * SZ, hd);
-      buf_store16(v1[u], wv, dst + v_off1 * SZ, hd);
+      if (lines) swap_lines(ok0, ok1);
+      buf_store16(ok0, wk, dst0 + ko0, hd);
+      buf_store16(ok1, wk, dst1 + ko1, hd);
+      buf_store16(v0[u], wv, dst0 + vo0, hd);
+      buf_store16(v1[u], wv, dst1 + vo1, hd);
     }
   }
 }
