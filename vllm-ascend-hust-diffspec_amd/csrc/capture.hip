@@ -92,8 +92,14 @@ __global__ __launch_bounds__(kThreadsC) void capture_kernel(CaptureArgs a) {
       const int h = e / vecs, c = e % vecs;
       const u32x4 kv = *reinterpret_cast<const u32x4*>(a.key + t * a.k_row + h * a.k_head + 16 * c);
       const u32x4 vv = *reinterpret_cast<const u32x4*>(a.value + t * a.v_row + h * a.v_head + 16 * c);
-      *reinterpret_cast<u32x4*>(a.raw_key + dst_row + static_cast<int64_t>(h) * a.row_bytes + 16 * c) = kv;
-      *reinterpret_cast<u32x4*>(a.raw_value + dst_row + static_cast<int64_t>(h) * a.row_bytes + 16 * c) = vv;
+      // Written once, read by a later gather: non-temporal stores.  us for 1 /
+      // 2 / 3 / 6 prompts of 8190 tokens (4 heads x 128, bf16): cached 7.1 /
+      // 13.5 / 20.0 / 41.8, non-temporal stores 7.0 / 12.0 / 16.9 / 33.7 (6.0
+      // TB/s), non-temporal loads too 8.2 / 13.5 / 19.3 / 35.5; 4 tokens per
+      // wave instead of one 7.5 / 12.2 / 18.0 / 35.6.
+      const int64_t dst = dst_row + static_cast<int64_t>(h) * a.row_bytes + 16 * c;
+      __builtin_nontemporal_store(kv, reinterpret_cast<u32x4*>(a.raw_key + dst));
+      __builtin_nontemporal_store(vv, reinterpret_cast<u32x4*>(a.raw_value + dst));
     }
   } else {  // rows that are not whole 16-byte vectors: element by element
     const int elems = a.row_bytes / a.elem;  // per head
