@@ -149,6 +149,42 @@ def test_whole_line_loads_give_the_bits_of_half_line_loads(cuda, head_dim, block
     assert torch.equal(out[0], out[1])
 
 
+@pytest.mark.parametrize("hkv,hq", [(1, 4), (2, 32), (4, 4), (8, 64), (16, 16), (3, 12)])
+@pytest.mark.parametrize("chunk,block_size", [(16, 16), (64, 40), (128, 128)])
+def test_every_kv_head_count_matches_oracle(cuda, hkv, hq, chunk, block_size):
+    # Spans of 1 to 16 KV heads in a workgroup's group of units (3 heads: two launches),
+    # empty rows and rows that end beside a chunk, tails past each row zero.
+    g = gen(21)
+    lengths = [0, 1, chunk - 1, chunk, chunk + 1, 777, 0, 2050, 63]
+    query = randn((len(lengths), hq, 64), torch.bfloat16, g)
+    key_cache, table = paged_keys(lengths, hkv, 64, block_size, torch.bfloat16, g)
+    lse = lse_for(query, key_cache, table, lengths, 0.125)
+    actual = _gpu_scores(query, key_cache, lse, table, lengths, chunk, 0.125, cuda)
+    expected = O.paged_chunk_attention_scores(query, key_cache, lse, table, torch.tensor(lengths), chunk_size=chunk,
+                                              max_seq_len=max(lengths), scale=0.125)
+    assert_scores_close(actual, expected)
+
+
+@pytest.mark.parametrize("hkv", [2, 16])
+def test_more_spans_than_a_segment(cuda, hkv):
+    # Several segments per workgroup: long rows whose block tables repeat four
+    # pages, one chunk each, so a chunk's score depends on its page alone.
+    g = gen(22)
+    query = randn((3, 16, 64), torch.bfloat16, g)
+    keys = randn((4, 64, hkv, 64), torch.bfloat16, g)
+    tokens = 400000 * 16 // hkv
+    lengths = [tokens, tokens - 64 * 5, tokens // 2]
+    pages = torch.randint(0, 4, (3, (tokens + 63) // 64), generator=g, dtype=torch.int32)
+    lse = torch.randn((3, 16), generator=g) + 8.0
+    actual = _gpu_scores(query, keys, lse, pages, lengths, 64, 0.125, cuda)
+    logits = torch.einsum("bhgd,pthd->bphgt", query.double().reshape(3, hkv, -1, 64), keys.double()) * 0.125
+    weights = (logits.reshape(3, 4, 16, 64) - lse.double()[:, None, :, None]).exp().mean((2, 3))
+    expected = torch.gather(weights, 1, pages.long()).float()
+    for b, n in enumerate(lengths):
+        expected[b, n // 64:] = 0.0
+    assert_scores_close(actual, expected)
+
+
 def test_headline_shape_scores(cuda):
     """16 requests, L ~ U[4096, 40960], 32 q heads / 4 KV heads x 128, chunk 64."""
     g = gen(0)

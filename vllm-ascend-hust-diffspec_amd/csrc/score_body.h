@@ -266,6 +266,20 @@ __device__ __forceinline__ void flush_mass(const ScoreArgs& a, const BatchCtx& c
   }
 }
 
+// LDS of a workgroup that writes final scores: the chunk sums of its last
+// kSegUnits units at most.  A group is kWaves units (a whole number of spans),
+// or the Hkv units of one span when Hkv is larger; wave w takes units w, w +
+// kWaves, ... of each of its workgroup's groups, so a span's heads meet in one
+// workgroup.  After every kSegUnits units (all waves' together) the workgroup
+// adds each span's heads and writes its scores: two LDS barriers, with the next
+// keys still in flight, in place of a second kernel.
+constexpr int kSegLog2 = 7;
+constexpr int kSegUnits = 1 << kSegLog2;
+constexpr int kFinalMaxHkv = 16;
+struct FinalShared {
+  float sum[kSegUnits][4];
+};
+
 // One wave's walk over its strided unit list: units gw, gw + tw, ... of the
 // numbering in s_prefix (rows' unit counts, exclusive prefix) with s_len /
 // s_qrow the rows' scored lengths and query rows.  Head mean stores
@@ -273,9 +287,13 @@ __device__ __forceinline__ void flush_mass(const ScoreArgs& a, const BatchCtx& c
 // max stores final chunk scores.  LSEFREE (head mean only): no LSE is read;
 // each chunk's mass word per query head goes to a.mw instead (tagged when
 // TAGGED).
-template <int DT, int STEPS, int KB, bool HMAX, int PAGE, bool TAGGED, bool LSEFREE = false>
+// FINAL (head mean, Hkv a power of two): units are dealt in groups (see
+// FinalShared), gw / tw are the workgroup's index and the grid, and the
+// workgroup writes the final scores itself.
+template <int DT, int STEPS, int KB, bool HMAX, int PAGE, bool TAGGED, bool LSEFREE = false, bool FINAL = false>
 __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_prefix, const int* s_len,
-                                             const int* s_qrow, int total, int gw, int tw, uint32_t tag) {
+                                             const int* s_qrow, int total, int gw, int tw, uint32_t tag,
+                                             FinalShared* fin = nullptr) {
   constexpr bool UNIFORM_PAGE = PAGE != PAGE_LANE;
   constexpr bool POW2 = PAGE == PAGE_POW2;
   constexpr bool LINES = UNIFORM_PAGE && STEPS % 2 == 0;  // whole-line key loads (swap_lines)
@@ -284,6 +302,38 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
   const int kgrp = lane >> 4;  // 8-element k slice of the 32-wide MFMA step
   const int bph = (a.ntu + KB - 1) / KB;     // batches per KV head of a unit
   const int bpu = bph * (HMAX ? a.Hkv : 1);  // batches per unit
+
+  // FINAL: groups of 1 << group_log2 units (whole spans), 1 << rounds_log2 of
+  // them per wave; the workgroup's groups make `flushes` segments.
+  const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
+  const int rounds_log2 = FINAL ? max(a.hkv_log2 - 2, 0) : 0;
+  const int group_log2 = rounds_log2 + 2;
+  const int seg_log2 = kSegLog2 - group_log2;  // groups per segment
+  int done = 0, flushed = 0;                   // units of this wave, segments
+  auto flush = [&]() {
+    lds_barrier();  // the segment's sums of all waves are in LDS
+    const int seg0 = flushed << seg_log2;
+    for (int i = threadIdx.x; i < (a.cpu << kSegLog2) >> a.hkv_log2; i += kThreads) {
+      const int span = i / a.cpu, cc = i - span * a.cpu;  // span within the segment
+      const int at = span << a.hkv_log2;                  // its head 0 within the segment
+      const int unit = ((gw + (seg0 + (at >> group_log2)) * tw) << group_log2) + (at & ((1 << group_log2) - 1));
+      if (unit >= total) continue;
+      int lo = 0, hi = a.batch - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_prefix[mid] <= unit) lo = mid; else hi = mid - 1;
+      }
+      const int ch = ((unit - s_prefix[lo]) >> a.hkv_log2) * a.cpu + cc;
+      const int n_valid = min(a.chunk, s_len[lo] - ch * a.chunk);
+      if (n_valid <= 0) continue;
+      float s = 0.f;  // heads in order, as finalize_kernel adds them
+      for (int g = 0; g < a.Hkv; ++g) s += fin->sum[at + g][cc];
+      a.out[static_cast<int64_t>(lo) * a.out_stride + ch] =
+          (s / static_cast<float>(n_valid)) / static_cast<float>(a.Hq);
+    }
+    lds_barrier();  // read before the next segment's sums overwrite it
+    ++flushed;
+  };
 
   // The wave's cursor: unit ordinal uk (unit gw + uk * tw), batch uj within
   // it, and for the head max the head hj and group batch tj within the
@@ -298,7 +348,11 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
   auto next_ctx = [&]() -> BatchCtx {
     if (uj == 0) {
       u = BatchCtx{};
-      const int unit = gw + uk * tw;
+      int unit = gw + uk * tw;
+      if constexpr (FINAL) {
+        const int round = uk & ((1 << rounds_log2) - 1);
+        unit = ((gw + (uk >> rounds_log2) * tw) << group_log2) + round * kWaves + wave;
+      }
       if (unit < total) {
         int lo = row_hint, hi = a.batch - 1;  // unit positions grow along the stream
         while (lo < hi) {
@@ -550,7 +604,10 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
         if (cc < a.cpu) {
           const float s = wave_sum_to_lane63(acc[cc]);
           const int ch = c.c0 + cc;
-          if (lane == 63 && ch < chunks_row) {
+          if constexpr (FINAL) {
+            const int k = done & ((1 << (kSegLog2 - 2)) - 1);  // kWaves units of the segment a round
+            if (lane == 63) fin->sum[k * kWaves + wave][cc] = s;
+          } else if (lane == 63 && ch < chunks_row) {
             const int64_t at = (static_cast<int64_t>(c.b) * a.max_chunks + ch) * a.Hkv + c.g;
             if constexpr (TAGGED) {
               // A coherent store that needs no wait: the value carries the
@@ -563,6 +620,9 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
           }
         }
         acc[cc] = 0.f;
+      }
+      if constexpr (FINAL) {
+        if ((++done & ((1 << (kSegLog2 - 2)) - 1)) == 0) flush();
       }
     }
   };
@@ -592,6 +652,13 @@ __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_pr
     pages_of(cx1, pg1);
     compute(d1);
     inherit(d0, d1);
+  }
+  if constexpr (FINAL) {
+    // Every wave of the workgroup flushes as often, whatever its own units.
+    const int groups = (total + (1 << group_log2) - 1) >> group_log2;
+    const int mine = groups > gw ? (groups - gw + tw - 1) / tw : 0;
+    const int flushes = (mine + (1 << seg_log2) - 1) >> seg_log2;
+    while (flushed < flushes) flush();
   }
 }
 

@@ -22,7 +22,8 @@
 // [row, chunk, KV head]; the head sum and the 1 / (Hq * n_valid)
 // normalisation (kernels.py:80-82, 150) happen where the partials are read:
 // in the selection kernel for a retrieval step, or in finalize_kernel for
-// the drop-in entry point.  The per-token head max (head_reduce = max) keeps
+// the drop-in entry point, unless the pass adds the heads itself in LDS
+// (FinalShared in score_body.h).  The per-token head max (head_reduce = max) keeps
 // all KV heads of a span in one wave and writes final scores directly.
 //
 // Without a supplied LSE (the reference's chunk_attention_scores with
@@ -47,8 +48,12 @@ using namespace score;
 // block-table lookups, one scalar lookup per group (block_size and the unit
 // start multiples of 16), or the same with power-of-two block size and KV
 // heads.
-template <int DT, int STEPS, int KB, int WGS, bool HMAX, int PAGE, bool LSEFREE>
+// OUT = what the pass writes: per-KV-head partials, the mass words (no LSE
+// supplied) or final scores.
+enum { OUT_PARTIAL, OUT_MASS, OUT_FINAL };
+template <int DT, int STEPS, int KB, int WGS, bool HMAX, int PAGE, int OUT>
 __global__ __launch_bounds__(kThreads, WGS) void chunk_score_kernel(ScoreArgs a) {
+  constexpr bool FINAL = OUT == OUT_FINAL;
   __shared__ int s_prefix[kMaxRows + 1];
   __shared__ int s_len[kMaxRows];
   __shared__ int s_qrow[kMaxRows];
@@ -64,12 +69,18 @@ __global__ __launch_bounds__(kThreads, WGS) void chunk_score_kernel(ScoreArgs a)
   build_row_prefix(a.batch, s_prefix, s_scratch,
                    [&](int r) { return (s_len[r] + a.U - 1) / a.U * units_per_span; });
   const int total = s_prefix[a.batch];
-  const int gw = uniform(blockIdx.x * kWaves + (threadIdx.x >> 6));
-  score_stream<DT, STEPS, KB, HMAX, PAGE, false, LSEFREE>(a, s_prefix, s_len, s_qrow, total, gw,
-                                                                  gridDim.x * kWaves, 0u);
+  if constexpr (FINAL) {
+    __shared__ FinalShared s_final;
+    score_stream<DT, STEPS, KB, false, PAGE, false, false, true>(a, s_prefix, s_len, s_qrow, total, blockIdx.x,
+                                                                 gridDim.x, 0u, &s_final);
+  } else {
+    const int gw = uniform(blockIdx.x * kWaves + (threadIdx.x >> 6));
+    score_stream<DT, STEPS, KB, HMAX, PAGE, false, OUT == OUT_MASS>(a, s_prefix, s_len, s_qrow, total, gw,
+                                                                    gridDim.x * kWaves, 0u);
+  }
 
   if (a.write_tail) {
-    // Head max writes final scores; chunks at or beyond a row's length are 0.
+    // Final scores: chunks at or beyond a row's length are 0.
     const int64_t n = static_cast<int64_t>(a.batch) * a.max_chunks;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n;
          i += static_cast<int64_t>(gridDim.x) * kThreads) {
@@ -200,7 +211,7 @@ __global__ __launch_bounds__(kThreads) void lse_finalize_kernel(const uint64_t* 
   }
 }
 
-template <int DT, int STEPS, bool HMAX, bool LSEFREE>
+template <int DT, int STEPS, bool HMAX, int OUT>
 void launch_kb(hipStream_t stream, const ScoreArgs& a, int64_t upper_blocks, int page_mode) {
   // Batch shape: about 4 KB of keys per wave and batch at three workgroups
   // per CU.  At head_dim 128 one 16-token group (4 KB) beat two (8 KB) by
@@ -221,25 +232,25 @@ void launch_kb(hipStream_t stream, const ScoreArgs& a, int64_t upper_blocks, int
   const int64_t cap = static_cast<int64_t>(device_cu_count()) * WGS;
   const int grid = static_cast<int>(std::max<int64_t>(1, std::min(upper_blocks, cap)));
   if (page_mode == PAGE_POW2) {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_POW2, LSEFREE><<<grid, kThreads, 0, stream>>>(a);
+    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_POW2, OUT><<<grid, kThreads, 0, stream>>>(a);
   } else if (page_mode == PAGE_UNIFORM) {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_UNIFORM, LSEFREE><<<grid, kThreads, 0, stream>>>(a);
+    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_UNIFORM, OUT><<<grid, kThreads, 0, stream>>>(a);
   } else {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_LANE, LSEFREE><<<grid, kThreads, 0, stream>>>(a);
+    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_LANE, OUT><<<grid, kThreads, 0, stream>>>(a);
   }
 }
 
-template <int DT, bool HMAX, bool LSEFREE>
+template <int DT, bool HMAX, int OUT>
 void launch_steps(hipStream_t stream, const ScoreArgs& a, int64_t grid, int page_mode) {
   switch (a.D / 32) {
-    case 1: launch_kb<DT, 1, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 2: launch_kb<DT, 2, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 3: launch_kb<DT, 3, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 4: launch_kb<DT, 4, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 5: launch_kb<DT, 5, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 6: launch_kb<DT, 6, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    case 7: launch_kb<DT, 7, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
-    default: launch_kb<DT, 8, HMAX, LSEFREE>(stream, a, grid, page_mode); break;
+    case 1: launch_kb<DT, 1, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 2: launch_kb<DT, 2, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 3: launch_kb<DT, 3, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 4: launch_kb<DT, 4, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 5: launch_kb<DT, 5, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 6: launch_kb<DT, 6, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 7: launch_kb<DT, 7, HMAX, OUT>(stream, a, grid, page_mode); break;
+    default: launch_kb<DT, 8, HMAX, OUT>(stream, a, grid, page_mode); break;
   }
 }
 
@@ -342,7 +353,7 @@ int make_score_args(ScoreArgs& a, int64_t& upper_units, int& page_mode, int dtyp
   a.mw = lse ? nullptr : mw;
   a.out = out;
   a.out_stride = out_stride;
-  a.write_tail = hmax ? write_tail : 0;
+  a.write_tail = write_tail;
 
   const int64_t spans = (static_cast<int64_t>(max_chunks) * chunk_size + U - 1) / U;
   upper_units = static_cast<int64_t>(batch) * spans * (hmax ? 1 : num_kv_heads);
@@ -361,7 +372,7 @@ int launch_chunk_scores(hipStream_t stream, int dtype, const void* query, int64_
                         int64_t bt_stride, const RowSource& src, int batch, int num_q_heads, int num_kv_heads,
                         int head_dim, int block_size, int chunk_size, int max_chunks, float scale, int head_reduce,
                         float* partial, float* out, int64_t out_stride, int write_tail, size_t partial_bytes,
-                        uint64_t* mw, float* lse_out, int64_t lse_out_stride) {
+                        uint64_t* mw, float* lse_out, int64_t lse_out_stride, bool final_out) {
   ScoreArgs a{};
   int64_t upper_units = 0;
   int page_mode = PAGE_LANE;
@@ -382,15 +393,19 @@ int launch_chunk_scores(hipStream_t stream, int dtype, const void* query, int64_
     DS_REQUIRE(lse_out_stride >= num_q_heads, "LSE output rows must hold every query head");
     DS_SUPPORTED(partial_grid < (int64_t{1} << 31), "too many (row, KV head, chunk slice) workgroups");
   }
-  const int64_t upper_blocks = (upper_units + kWaves - 1) / kWaves;
+  // Groups of units for final scores (FinalShared): kWaves units, or one span's Hkv.
+  const int group = final_out ? std::max(kWaves, num_kv_heads) : kWaves;
+  const int64_t upper_blocks = (upper_units + group - 1) / group;
   if (dtype == DS_BF16) {
-    if (hmax) launch_steps<DS_BF16, true, false>(stream, a, upper_blocks, page_mode);
-    else if (lse_free) launch_steps<DS_BF16, false, true>(stream, a, upper_blocks, page_mode);
-    else launch_steps<DS_BF16, false, false>(stream, a, upper_blocks, page_mode);
+    if (hmax) launch_steps<DS_BF16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
+    else if (lse_free) launch_steps<DS_BF16, false, OUT_MASS>(stream, a, upper_blocks, page_mode);
+    else if (final_out) launch_steps<DS_BF16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode);
+    else launch_steps<DS_BF16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
   } else {
-    if (hmax) launch_steps<DS_FP16, true, false>(stream, a, upper_blocks, page_mode);
-    else if (lse_free) launch_steps<DS_FP16, false, true>(stream, a, upper_blocks, page_mode);
-    else launch_steps<DS_FP16, false, false>(stream, a, upper_blocks, page_mode);
+    if (hmax) launch_steps<DS_FP16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
+    else if (lse_free) launch_steps<DS_FP16, false, OUT_MASS>(stream, a, upper_blocks, page_mode);
+    else if (final_out) launch_steps<DS_FP16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode);
+    else launch_steps<DS_FP16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
   }
   int rc2 = check_launch("ds_chunk_scores");
   if (rc2 != DS_OK || !lse_free) return rc2;
@@ -433,11 +448,20 @@ extern "C" int ds_chunk_scores(ds_stream_t stream, int dtype, const void* query,
       partial_bytes = workspace_bytes - (pairs + lses) * sizeof(float);
     }
   }
+  // The pass adds the heads and writes the scores itself when a span's KV
+  // heads fill a workgroup's waves evenly (a power of two); otherwise, and
+  // without an LSE, finalize_kernel does.  us with one / two launches: 8 rows of
+  // 900-16k tokens (32/8 heads x 64) 13.7 / 15.7, one of 300 (32/4 x 128) 6.2 /
+  // 7.4, 16 of 4-40k (32/4 x 128) 63.1 / 64.9, 16 of 4-20k (16/16 x 64) 61.1 /
+  // 66.8, 16 of 4-40k (32/8 x 64, 16-token chunks) 66.7 / 75.8.
+  const bool final_out = lse != nullptr && !hmax && out != nullptr && num_kv_heads > 0 &&
+                         num_kv_heads <= kFinalMaxHkv && (num_kv_heads & (num_kv_heads - 1)) == 0;
   int rc = launch_chunk_scores(s, dtype, query, q_stride, key_cache, k_block_stride, k_token_stride, k_head_stride,
                                lse, lse_row_stride, lse_head_stride, block_table, bt_stride, src, batch, num_q_heads,
                                num_kv_heads, head_dim, block_size, chunk_size, max_chunks, scale, head_reduce,
-                               partial, out, out_stride, 1, partial_bytes, mw, lse_rows, num_q_heads);
-  if (rc != DS_OK || hmax || batch == 0 || max_chunks == 0) return rc;
+                               partial, out, out_stride, hmax || final_out ? 1 : 0, partial_bytes, mw, lse_rows,
+                               num_q_heads, final_out);
+  if (rc != DS_OK || hmax || batch == 0 || max_chunks == 0 || final_out) return rc;
   DS_REQUIRE(out != nullptr, "null score output pointer");
   const int64_t n = static_cast<int64_t>(batch) * max_chunks;
   const int grid = static_cast<int>(std::min<int64_t>((n + kThreads - 1) / kThreads, 4096));

@@ -16,7 +16,7 @@ int launch_chunk_scores(hipStream_t stream, int dtype, const void* query, int64_
                         int64_t bt_stride, const RowSource& src, int batch, int num_q_heads, int num_kv_heads,
                         int head_dim, int block_size, int chunk_size, int max_chunks, float scale, int head_reduce,
                         float* partial, float* out, int64_t out_stride, int write_tail, size_t partial_bytes,
-                        uint64_t* mw, float* lse_out, int64_t lse_out_stride);
+                        uint64_t* mw, float* lse_out, int64_t lse_out_stride, bool final_out);
 
 int launch_select_plan(hipStream_t stream, float* scores, int64_t score_stride, const float* partials,
                        int max_chunks, int hkv, int hq, const RowSource& src,
@@ -104,7 +104,7 @@ int retrieval_step(hipStream_t stream, const ds_step_desc* d, uint32_t* status_o
                              d->block_table, d->bt_stride, src, d->batch_rows, d->num_q_heads, d->num_kv_heads,
                              d->head_dim, d->block_size, d->chunk_size, d->max_chunks, d->scale, DS_HEAD_MEAN,
                              d->score_partials, nullptr, 0, 0, SIZE_MAX, reinterpret_cast<uint64_t*>(d->lse_partials), d->lse_out,
-                             d->lse_out_stride);
+                             d->lse_out_stride, false);
     if (rc != DS_OK) return rc;
   }
   // The rebuild as one plan + gather launch (the compact prefill's kernel)
