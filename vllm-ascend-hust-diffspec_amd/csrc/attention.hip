@@ -135,17 +135,18 @@ __device__ __forceinline__ float unpack(uint32_t w, int half) {
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
-// Working rows are read in whole 128-byte lines, non-temporally (a bare read
-// loop on this card: 5.95 TB/s cached or in half lines, 6.7-6.9 TB/s so).  The
-// A operand of the score MFMAs wants 64 bytes of each of 16 tokens (lane quad
-// * 16 + col: token col, 16-byte slice quad).  Loads 2 p and 2 p + 1 of a tile
-// therefore take line p of tokens 0-7 and of tokens 8-15: lane (quad, col)
-// holds slice quad + 4 (col / 8) of token (col % 8) + 8 (i % 2), and
-// swap_lines exchanges halves between lanes col and col ^ 8.
+// Working rows are read in whole 128-byte lines.  The A operand of the score
+// MFMAs wants 64 bytes of each of 16 tokens (lane quad * 16 + col: token col,
+// 16-byte slice quad).  Loads 2 p and 2 p + 1 of a tile therefore take line p
+// of tokens 0-7 and of tokens 8-15: lane (quad, col) holds slice quad + 4 (col
+// / 8) of token (col % 8) + 8 (i % 2), and swap_lines exchanges halves between
+// lanes col and col ^ 8.  attention_stream_kernel, whose batches come from
+// HBM, loads them non-temporally (a bare read loop on this card: 5.95 TB/s
+// cached or in half lines, 6.7-6.9 TB/s so).  A one-round batch fits the 256
+// MB last-level cache and is read again in the next draft step: cached loads
+// there (16 rows of 1987: 16.5 us, non-temporal 17.0; a 16-row draft cycle
+// 181.5 against 185.7).
 constexpr int kPolicyNt = 2;
-__device__ __forceinline__ u32x4 load16_nt(const uint16_t* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-}
 __device__ __forceinline__ int line_token(int col, int i) { return (col & 7) + 8 * (i & 1); }
 __device__ __forceinline__ int line_elem(int quad, int col, int i) { return 8 * quad + 32 * (col >> 3) + 64 * (i >> 1); }
 constexpr int kRowRor8 = 0x128;  // DPP: lane c of a 16-lane row reads lane c ^ 8
@@ -184,16 +185,15 @@ template <int J>
 __device__ __forceinline__ constexpr int v_elem(int m) { return (J < 8 ? J : 8) * m; }
 template <int J>
 __device__ __forceinline__ constexpr int out_dim(int m, int j) { return v_elem<J>(m) + (j & 7) + (j >> 3) * 128; }
-template <int J, bool NT>
+template <int J>
 __device__ __forceinline__ void load_words(const uint16_t* p, uint32_t (&w)[J / 2]) {
   if constexpr (J == 4) {
-    const u32x2 v = NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p))
-                       : *reinterpret_cast<const u32x2*>(p);
+    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
     w[0] = v.x; w[1] = v.y;
   } else {
 #pragma unroll
     for (int h = 0; h < J / 8; ++h) {
-      const u32x4 v = NT ? load16_nt(p + 128 * h) : load16(p + 128 * h);
+      const u32x4 v = load16(p + 128 * h);
       w[4 * h] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
     }
   }
@@ -614,12 +614,12 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
 #pragma unroll
       for (int i = 0; i < S::kSteps; ++i) {
         const int t = min(tb + h * kTileT + line_token(col, i), a.budget - 1);
-        K.k[h][i] = load16_nt(kw + static_cast<int64_t>(t) * D + line_elem(quad, col, i));
+        K.k[h][i] = load16(kw + static_cast<int64_t>(t) * D + line_elem(quad, col, i));
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = min(tb + h * kTileT + 4 * quad + r, a.budget - 1);
-        load_words<J, true>(vw + static_cast<int64_t>(t) * D + v_elem<J>(col), V.v[h][r]);
+        load_words<J>(vw + static_cast<int64_t>(t) * D + v_elem<J>(col), V.v[h][r]);
       }
     }
   };
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
     load_rows(k0, v0, t0);
 #pragma unroll
     for (int i = 0; i < S::kSteps; i += 2) kin_s[i / 2] = load16(kin + line_elem(quad, col, i));
-    load_words<J, false>(vin + v_elem<J>(col), vin_s);
+    load_words<J>(vin + v_elem<J>(col), vin_s);
   }
   lds_barrier();
   const int pos = s_pos;
@@ -693,11 +693,11 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
       for (int i = 0; i < S::kSteps; ++i) {
-        K.k[h][i] = load16_nt(row_ptr(kw, kin, tb + h * kTileT + line_token(col, i)) + line_elem(quad, col, i));
+        K.k[h][i] = load16(row_ptr(kw, kin, tb + h * kTileT + line_token(col, i)) + line_elem(quad, col, i));
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        load_words<J, true>(row_ptr(vw, vin, tb + h * kTileT + 4 * quad + r) + v_elem<J>(col), V.v[h][r]);
+        load_words<J>(row_ptr(vw, vin, tb + h * kTileT + 4 * quad + r) + v_elem<J>(col), V.v[h][r]);
       }
     }
   };
@@ -950,7 +950,7 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int t = tb + h * kTileT + 4 * quad + r;
-          load_words<J, false>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + v_elem<J>(col), T.v[h][r]);
+          load_words<J>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + v_elem<J>(col), T.v[h][r]);
         }
       }
     }
