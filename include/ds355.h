@@ -362,7 +362,9 @@ int ds_retrieval_step_static(ds_stream_t stream, const ds_step_desc* desc, uint3
  *          256-byte aligned; reused across launches (one stream at a time).
  *          Word 2 of its header is the status word (bit 1: the wait of the
  *          last workgroup for the others' "seen" words expired: that
- *          launch's working lengths were not advanced).
+ *          launch's working lengths were not advanced; its outputs and
+ *          cache rows are written).  Word 3, set nonzero by the owner, ends
+ *          that wait at once (tests of this).
  * One kernel launch, no host synchronisation, fixed launch shape for the
  * given sizes (graph-capturable).
  */
@@ -383,7 +385,7 @@ int ds_draft_attention(ds_stream_t stream, int dtype,
  * counterpart.  With U = batch_rows x Hkv x ceil(G / 16) row units (at most
  * 65536) and W = U x ceil(token_budget / span) workgroups (span = 256
  * tokens, 128 for head_dim 256): 256 header bytes (word 0 the epoch, word 2
- * the status), 65536 4-byte span counters (0 between launches, at a fixed
+ * the status, word 3 the owner's), 65536 4-byte span counters (0 between launches, at a fixed
  * place for every shape), W 8-byte tagged "seen" words rounded up to 256
  * bytes, then W x 16 x (head_dim + 4) fp32 partial results.
  */

@@ -324,3 +324,34 @@ def test_streamed_batches(cuda, rows, hq, hkv, dim, budget, dtype):
     terms = attention_terms(q, k_all, v_all, slots, [n + 3 for n in lengths], dim ** -0.5)
     assert_attention_close(partly[keep], whole[keep], terms[keep])  # other range ends: sums in another order
     assert attention.attention_status(dev.ws) == attention.STATUS_BAD_POSITION
+
+
+@pytest.mark.parametrize("rows,dim,budget", [(3, 128, 512), (20, 128, 2048)])
+def test_expired_wait_keeps_the_working_lengths(cuda, rows, dim, budget):
+    """A launch whose last workgroup stops waiting for the others (forced by the owner's header
+    word) sets bit 1 and leaves the working lengths, in the one-shot and the streamed kernel; its
+    outputs and cache rows are written, and the next launch on the workspace is an ordinary one."""
+    from ds355 import attention
+
+    case = Case(rows + dim, rows, 4, 32, dim, budget)
+    for s in range(rows):
+        case.fill(s, (97 * s + 40) % (budget - 2))
+    dev = Device(case, cuda, rows)
+    slots, positions = list(range(rows)), case.lens.tolist()
+    q, k, v = case.inputs(rows)
+    dev.ws[12:16].view(torch.int32).fill_(1)
+    out = torch.full_like(q, float("nan")).to(cuda)
+    attention.draft_linear_attention(q.to(cuda), k.to(cuda), v.to(cuda), out, dev.k, dev.v, dev.lens, slots, None,
+                                     scale=0.1, workspace=dev.ws)
+    torch.cuda.synchronize()
+    assert attention.attention_status(dev.ws) == attention.STATUS_PARTIAL_TIMEOUT
+    assert attention.attention_epoch(dev.ws) == 1
+    assert torch.equal(dev.lens.cpu(), case.lens)
+    expected = torch.zeros_like(q)
+    O.draft_linear_attention(q, k, v, 0.1, expected, case.work_k, case.work_v, case.lens.tolist(), slots, positions)
+    assert_attention_close(out.cpu(), expected, attention_terms(q, case.work_k, case.work_v, slots, positions, 0.1))
+    _same_bits(dev.k.cpu(), case.work_k)
+    _same_bits(dev.v.cpu(), case.work_v)
+    dev.ws[8:16].view(torch.int32).zero_()
+    _step(case, dev, cuda, slots, None, rows, 0.1)
+    assert attention.attention_epoch(dev.ws) == 2

@@ -77,10 +77,10 @@ constexpr float kLog2e = 1.44269504088896340736f;
 // results of every span.
 constexpr int kMaxUnits = 65536;
 constexpr size_t kCounterBytes = kMaxUnits * sizeof(uint32_t);
-enum { kHdrEpoch = 0, kHdrStatus = 2 };
+enum { kHdrEpoch = 0, kHdrStatus = 2, kHdrGiveUp = 3 };  // kHdrGiveUp: set by the owner, the wait ends at once
 constexpr size_t kHeaderBytes = 256;
 constexpr uint32_t kStatusPosition = 1;  // a row's slot or position was out of range
-constexpr uint32_t kStatusPartials = 2;  // a merge stopped waiting for a partial
+constexpr uint32_t kStatusExpired = 2;   // the last workgroup stopped waiting for the others
 
 template <int D>
 struct AttnShape {
@@ -242,23 +242,19 @@ __device__ __forceinline__ void raise_status(const AttnArgs& a, uint32_t bit) {
   __hip_atomic_fetch_or(a.header + kHdrStatus, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Value of a tagged partial word once its tag is this launch's.  The writer
-// counted itself after issuing the store, so the wait is for a store in
-// flight; it is bounded all the same, and after one expiry the thread stops
-// waiting (NaN results, status bit set).
-__device__ __forceinline__ float settle(const AttnArgs& a, const uint64_t* p, uint64_t v, uint32_t tag,
-                                        bool& expired) {
+// Waits until a workgroup's seen word carries this launch's tag.  The wait is
+// bounded: after one expiry the thread stops waiting (status bit set).
+__device__ __forceinline__ void await_seen(const AttnArgs& a, const uint64_t* p, uint32_t tag, bool& expired) {
   uint32_t spins = 0;
-  while (static_cast<uint32_t>(v >> 32) != tag) {
-    if (expired || ++spins > kSpinA) {
-      if (!expired) raise_status(a, kStatusPartials);
+  for (uint64_t v = coherent_load(p); static_cast<uint32_t>(v >> 32) != tag; v = coherent_load(p)) {
+    if (expired) return;
+    if (++spins > kSpinA) {
+      raise_status(a, kStatusExpired);
       expired = true;
-      return __uint_as_float(0x7fc00000u);
+      return;
     }
     __builtin_amdgcn_s_sleep(2);
-    v = coherent_load(p);
   }
-  return __uint_as_float(static_cast<uint32_t>(v));
 }
 
 // Zero out[row, head0 .. head0 + count) (padding rows and rows with a bad position).
@@ -540,19 +536,29 @@ __device__ __forceinline__ void write_token(const AttnArgs& a, int64_t work_base
 // Run by the grid's last workgroup at its end: once every workgroup of the
 // pending rows has stored its seen word (all of them have lower indices and
 // were dispatched before this one), each row's working length becomes
-// position + 1 and the epoch advances.
+// position + 1 and the epoch advances.  If that wait expires (on any thread),
+// a workgroup may still have its position to read: the working lengths stay
+// as they are.  The epoch advances all the same, or the next launch would
+// take this one's seen words for its own.
 __device__ __forceinline__ void publish(const AttnArgs& a, uint32_t tag, int seen_words) {
-  bool expired = false;
+  __shared__ int s_expired[kWavesA];
+  bool expired = coherent_load(a.header + kHdrGiveUp) != 0u;
+  if (expired && threadIdx.x == 0) raise_status(a, kStatusExpired);
   for (int b = threadIdx.x; b < seen_words; b += kThreadsA) {
-    if (b != static_cast<int>(blockIdx.x)) settle(a, a.seen + b, coherent_load(a.seen + b), tag, expired);
+    if (b != static_cast<int>(blockIdx.x)) await_seen(a, a.seen + b, tag, expired);
   }
+  const bool wave_expired = __any(expired);
+  if ((threadIdx.x & 63) == 0) s_expired[threadIdx.x >> 6] = wave_expired ? 1 : 0;
   lds_barrier();
+  int give_up = 0;
+#pragma unroll
+  for (int w = 0; w < kWavesA; ++w) give_up |= s_expired[w];
   for (int r = threadIdx.x; r < a.rows; r += kThreadsA) {
     const int slot = a.slots[r];
     int pos = -1;
     if (slot >= 0 && slot < a.num_slots) pos = a.positions ? a.positions[r] : a.working_lens[slot];
-    if (pos >= 0 && pos < a.budget) a.working_lens[slot] = pos + 1;
-    else raise_status(a, kStatusPosition);
+    if (pos < 0 || pos >= a.budget) raise_status(a, kStatusPosition);
+    else if (give_up == 0) a.working_lens[slot] = pos + 1;
   }
   if (threadIdx.x == 0 && a.rows > 0) coherent_store(a.header + kHdrEpoch, tag);
 }

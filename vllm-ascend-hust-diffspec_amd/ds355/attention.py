@@ -48,12 +48,13 @@ def new_attention_workspace(batch_rows: int, num_q_heads: int, num_kv_heads: int
 def attention_status(workspace: torch.Tensor) -> int:
     """Status word (reads the device): bit 0 a row's slot or position was out
     of range, bit 1 the last workgroup's wait for the others' "seen" words
-    expired (that launch did not advance the working lengths)."""
+    expired (that launch did not advance the working lengths; its outputs and
+    cache rows are written)."""
     return int(workspace[8:12].view(torch.int32).item())
 
 
 def attention_epoch(workspace: torch.Tensor) -> int:
-    """Launches completed on this workspace that had at least one pending row."""
+    """Launches completed on this workspace that had at least one pending row (an expired wait among them)."""
     return int(workspace[0:4].view(torch.int32).item())
 
 
