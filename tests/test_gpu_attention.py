@@ -355,3 +355,36 @@ def test_expired_wait_keeps_the_working_lengths(cuda, rows, dim, budget):
     dev.ws[8:16].view(torch.int32).zero_()
     _step(case, dev, cuda, slots, None, rows, 0.1)
     assert attention.attention_epoch(dev.ws) == 2
+
+
+@pytest.mark.parametrize("rows,budget,inside", [
+    (6, 512, [8, 14, 15, 16, 25, 30]),  # one-shot: the first tile pair of each wave's four
+    (40, 2048, [8, 14, 15, 16, 25, 30, 31, 40, 47, 48, 60, 63])])  # streamed
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_infinite_value_of_the_new_token(cuda, rows, budget, inside, dim):
+    """An infinity in the new token's value stays that infinity in its output column, wherever the
+    token lies within a wave's tiles: it is also loaded in place of rows past the position, with
+    probability 0, and must not become NaN there.  Other tokens of the pair come first, so the new
+    one is not its maximum.  bf16, whose probabilities split into two parts of one sign (fp16's
+    lower part may be negative)."""
+    from ds355 import attention
+
+    case = Case(rows * dim, rows, 4, 16, dim, budget)
+    positions = [64 * (5 * r % (budget // 64)) + inside[r % len(inside)] for r in range(rows)]
+    for s, n in enumerate(positions):
+        case.fill(s, n)
+    q, k, v = case.inputs(rows)
+    k.zero_()  # a score of 0, below the maximum: both parts of the probability are above 0
+    v[:, :, 5], v[:, :, dim - 3] = float("inf"), float("-inf")
+    dev = Device(case, cuda, rows)
+    out = torch.full_like(q, float("nan")).to(cuda)
+    attention.draft_linear_attention(q.to(cuda), k.to(cuda), v.to(cuda), out, dev.k, dev.v, dev.lens,
+                                     list(range(rows)), None, scale=dim ** -0.5, workspace=dev.ws)
+    expected = torch.zeros_like(q)
+    O.draft_linear_attention(q, k, v, dim ** -0.5, expected, case.work_k, case.work_v, case.lens.tolist(),
+                             list(range(rows)), positions)
+    actual = out.cpu()
+    assert not expected.isnan().any() and (expected[:, :, 5] == float("inf")).all()
+    for name in ("isnan", "isposinf", "isneginf"):
+        differ = (getattr(torch, name)(actual) != getattr(torch, name)(expected)).nonzero().tolist()
+        assert not differ, (name, differ[:4])

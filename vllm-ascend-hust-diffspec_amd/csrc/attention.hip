@@ -312,6 +312,23 @@ __device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv
   }
 }
 
+// V rows past the position (of the 32 tokens from tb on) become zeros: their
+// probabilities are 0, and 0 times an infinity of the new token's row, which
+// is loaded in their place, would not be.
+template <int D>
+__device__ __forceinline__ void zero_past(VTiles<D>& T, int tb, int pos, int quad) {
+  if (tb + 2 * kTileT <= pos + 1) return;  // wave-uniform
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const bool past = tb + h * kTileT + 4 * quad + r > pos;
+#pragma unroll
+      for (int w = 0; w < AttnShape<D>::kJ / 2; ++w) T.v[h][r][w] = past ? 0u : T.v[h][r][w];
+    }
+  }
+}
+
 // Online softmax and output of the 32 tokens tb .. tb + 31 (n valid tokens in
 // all).  The output MFMAs are 16x16x32 in the cache dtype with A = V^T and
 // B = P^T: k-slot (lane / 16, e) is token 4 * (lane / 16) + (e & 3) of tile
@@ -997,7 +1014,10 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
       __builtin_amdgcn_sched_barrier(0);
       if (more) load_k(K, u, tb + kStep);
       __builtin_amdgcn_sched_barrier(0);
-      if (tb < n) pair_output<DT, D>(V, sc, run, tb, n, quad, c);
+      if (tb < n) {
+        zero_past<D>(V, tb, u.pos, quad);
+        pair_output<DT, D>(V, sc, run, tb, n, quad, c);
+      }
       __builtin_amdgcn_sched_barrier(0);
       if (!more) break;
       tb += kStep;
