@@ -344,6 +344,8 @@ int ds_retrieval_step_static(ds_stream_t stream, const ds_step_desc* desc, uint3
  *                uses KV head hq / G, the reference's repeat_interleave),
  *                scores, softmax and the weighted sum in fp32, rounded once
  *                to the output dtype;
+ * a row's bits depend on that row alone, not on the rows beside it or their
+ * number;
  * rows rows <= r < out_rows of `out` are written as zeros (the reference's
  * output.zero_() for graph padding).  A row whose slot or position is out
  * of range ([0, num_slots), [0, token_budget)) gets zeros, changes nothing

@@ -317,12 +317,11 @@ def test_streamed_batches(cuda, rows, hq, hkv, dim, budget, dtype):
         chosen = [-1 if r == bad else s for r, s in enumerate(slots)]
         attention.draft_linear_attention(q.to(cuda), k.to(cuda), v.to(cuda), out, k_dev, v_dev, lens, chosen, None,
                                          scale=dim ** -0.5, workspace=dev.ws)
-        outs.append((out.cpu(), k_dev.cpu(), v_dev.cpu()))
+        outs.append(out.cpu())
     keep = [r for r in range(rows) if r != rows // 2]
-    (whole, k_all, v_all), (partly, _, _) = outs
+    whole, partly = outs
     assert partly[rows // 2].count_nonzero() == 0
-    terms = attention_terms(q, k_all, v_all, slots, [n + 3 for n in lengths], dim ** -0.5)
-    assert_attention_close(partly[keep], whole[keep], terms[keep])  # other range ends: sums in another order
+    _same_bits(partly[keep], whole[keep])
     assert attention.attention_status(dev.ws) == attention.STATUS_BAD_POSITION
 
 
@@ -364,9 +363,8 @@ def test_expired_wait_keeps_the_working_lengths(cuda, rows, dim, budget):
 def test_infinite_value_of_the_new_token(cuda, rows, budget, inside, dim):
     """An infinity in the new token's value stays that infinity in its output column, wherever the
     token lies within a wave's tiles: it is also loaded in place of rows past the position, with
-    probability 0, and must not become NaN there.  Other tokens of the pair come first, so the new
-    one is not its maximum.  bf16, whose probabilities split into two parts of one sign (fp16's
-    lower part may be negative)."""
+    probability 0, and must not become NaN there.  bf16, whose probabilities split into two
+    parts of one sign (fp16's lower part may be negative)."""
     from ds355 import attention
 
     case = Case(rows * dim, rows, 4, 16, dim, budget)
@@ -374,7 +372,9 @@ def test_infinite_value_of_the_new_token(cuda, rows, budget, inside, dim):
     for s, n in enumerate(positions):
         case.fill(s, n)
     q, k, v = case.inputs(rows)
-    k.zero_()  # a score of 0, below the maximum: both parts of the probability are above 0
+    q.abs_()
+    case.work_k[:, :, ::8].abs_()  # scores above 0 in every half tile; the new token's is 0,
+    k.zero_()  # so both parts of its probability are above 0
     v[:, :, 5], v[:, :, dim - 3] = float("inf"), float("-inf")
     dev = Device(case, cuda, rows)
     out = torch.full_like(q, float("nan")).to(cuda)
@@ -388,3 +388,55 @@ def test_infinite_value_of_the_new_token(cuda, rows, budget, inside, dim):
     for name in ("isnan", "isposinf", "isneginf"):
         differ = (getattr(torch, name)(actual) != getattr(torch, name)(expected)).nonzero().tolist()
         assert not differ, (name, differ[:4])
+
+
+def _launched_streamed(ws, rows, hkv, group, dim, budget, tag):
+    """Whether the launch of epoch `tag` was the streamed kernel: its workgroups, fewer than the
+    batch's spans, are the ones that leave "seen" words."""
+    spans = rows * hkv * ((group + 15) // 16) * (-(-budget // (256 if dim <= 128 else 128)))
+    seen = ws[256 + 4 * 65536:][: 8 * spans].view(torch.int32)[1::2]
+    return int((seen == tag).sum()) < spans
+
+
+@pytest.mark.parametrize("rows,hq,hkv,dim,budget,dtype", [
+    (24, 32, 4, 128, 2048, torch.bfloat16),  # one query block, units within and across ranges
+    (57, 64, 8, 128, 4096, torch.float16),
+    (48, 32, 8, 64, 2048, torch.bfloat16),
+    (16, 64, 2, 256, 2048, torch.bfloat16),  # two query blocks
+    (7, 16, 1, 256, 8192, torch.float16),  # fewer units than workgroups: units of many ranges
+])
+def test_a_row_has_the_same_bits_in_any_batch(cuda, rows, hq, hkv, dim, budget, dtype):
+    """A row's output does not depend on the rows beside it, their order or count, nor on which
+    kernel the batch's size selects: a streamed batch, its reverse, a part of it and every row
+    alone (one-shot) give the same bits."""
+    from ds355 import attention
+
+    case = Case(rows + dim, rows, hkv, hq, dim, budget, dtype)
+    edges = [0, 31, 127, 128, 255, 256, 511, 700, budget // 2, budget - 130, budget - 1]
+    positions = [min(edges[(3 * r) % len(edges)] + r // len(edges), budget - 1) for r in range(rows)]
+    case.work_k, case.work_v = (randn(case.shape, dtype, case.g) for _ in range(2))
+    dev = Device(case, cuda, rows)
+    q, k, v = (t.to(cuda) for t in case.inputs(rows))
+
+    def run(order):
+        at = torch.tensor(order, device=cuda)
+        out = torch.empty((len(order), hq, dim), dtype=dtype, device=cuda)
+        attention.draft_linear_attention(q[at], k[at], v[at], out, dev.k, dev.v, dev.lens, order,
+                                         [positions[r] for r in order], scale=dim ** -0.5, workspace=dev.ws)
+        torch.cuda.synchronize()
+        streamed = _launched_streamed(dev.ws, len(order), hkv, hq // hkv, dim, budget,
+                                      attention.attention_epoch(dev.ws))
+        return out.cpu(), streamed
+
+    whole, streamed = run(list(range(rows)))
+    assert streamed
+    backwards, streamed = run(list(range(rows))[::-1])
+    assert streamed
+    _same_bits(backwards.flip(0), whole)
+    part, _ = run(list(range(1, rows, 2)))
+    _same_bits(part, whole[1::2])
+    for r in range(rows):
+        alone, streamed = run([r])
+        assert not streamed
+        _same_bits(alone[0], whole[r])
+    assert attention.attention_status(dev.ws) == 0

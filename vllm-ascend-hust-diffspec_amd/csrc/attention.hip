@@ -208,15 +208,14 @@ constexpr int kPolicySc1 = 16;
 __device__ __forceinline__ Rsrc16 make_rsrc16(const void* base, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
 }
-__device__ __forceinline__ void store16_sc1(Rsrc16 r, uint32_t off, f32x4 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, static_cast<int>(off), 0, kPolicySc1);
+__device__ __forceinline__ void store16_sc1(Rsrc16 r, int voff, int soff, f32x4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, kPolicySc1);
 }
-__device__ __forceinline__ f32x4 load16_sc1(Rsrc16 r, uint32_t off) {
-  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, kPolicySc1));
+__device__ __forceinline__ f32x4 load16_sc1(Rsrc16 r, int voff, int soff) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kPolicySc1));
 }
-
-__device__ __forceinline__ f32x2 load8_sc1(Rsrc16 r, uint32_t off) {
-  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(off), 0, kPolicySc1));
+__device__ __forceinline__ f32x2 load8_sc1(Rsrc16 r, int voff, int soff) {
+  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kPolicySc1));
 }
 
 // The same through a buffer resource, non-temporally.
@@ -312,23 +311,6 @@ __device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv
   }
 }
 
-// V rows past the position (of the 32 tokens from tb on) become zeros: their
-// probabilities are 0, and 0 times an infinity of the new token's row, which
-// is loaded in their place, would not be.
-template <int D>
-__device__ __forceinline__ void zero_past(VTiles<D>& T, int tb, int pos, int quad) {
-  if (tb + 2 * kTileT <= pos + 1) return;  // wave-uniform
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool past = tb + h * kTileT + 4 * quad + r > pos;
-#pragma unroll
-      for (int w = 0; w < AttnShape<D>::kJ / 2; ++w) T.v[h][r][w] = past ? 0u : T.v[h][r][w];
-    }
-  }
-}
-
 // Online softmax and output of the 32 tokens tb .. tb + 31 (n valid tokens in
 // all).  The output MFMAs are 16x16x32 in the cache dtype with A = V^T and
 // B = P^T: k-slot (lane / 16, e) is token 4 * (lane / 16) + (e & 3) of tile
@@ -391,13 +373,15 @@ struct MergeShared {
   float l[kWavesA][kGroupQ];
 };
 
-// The waves' states go to LDS as they are (then a barrier).
+// The waves' states of `gcount` queries go to LDS as they are (then a barrier).
 template <int D>
-__device__ __forceinline__ void waves_to_lds(MergeShared<D>& sh, const Running<D>& run, int wave, int quad, int col) {
+__device__ __forceinline__ void waves_to_lds(MergeShared<D>& sh, const Running<D>& run, int wave, int quad, int col,
+                                             int gcount) {
   constexpr int J = AttnShape<D>::kJ;
   float l = run.l;
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  if (col >= gcount) return;
   if (quad == 0) {
     sh.m[wave][col] = run.m;
     sh.l[wave][col] = l;
@@ -451,26 +435,38 @@ __device__ __forceinline__ void write_outputs(const AttnArgs& a, const MergeShar
   }
 }
 
-// A unit done by several workgroups: this one's partial ((running max, sum,
-// unnormalised output) per query, fp32) goes to its place `off` (bytes) of
-// the partials with device-scope stores, which are waited for; then the
-// workgroup counts itself on the unit's counter.  True for the one that
-// counts last of `parts`: the others' stores are complete before their
-// counts, so it can read them without waiting, and it resets the counter for
-// the next launch.
-template <int D>
-__device__ __forceinline__ bool count_partial(const AttnArgs& a, const MergeShared<D>& sh, Rsrc16 prs, uint32_t off,
-                                              int gcount, int unit, int parts, int* s_last, int tid) {
-  using S = AttnShape<D>;
-  constexpr int kChunks = D / 4;
-  // Row g of a partial: D outputs, then (max, sum, 0, 0).
-  for (int item = tid; item < gcount * kChunks; item += kThreadsA) {
-    const int g = item / kChunks, e = 4 * (item % kChunks);
-    float mx, total_l;
-    const f32x4 v = span_item<D>(sh, g, e, mx, total_l);
-    store16_sc1(prs, off + static_cast<uint32_t>((g * S::kRow + e) * 4), v);
-    if (e == 0) store16_sc1(prs, off + static_cast<uint32_t>((g * S::kRow + D) * 4), f32x4{mx, total_l, 0.f, 0.f});
+// One more span joins a query's running (max, sum, outputs): the spans of a
+// row are merged in index order by this one expression, whichever workgroup
+// and kernel does it, so a row's result depends on that row alone.
+struct Merged {
+  float m = -INFINITY, l = 0.f;
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  __device__ __forceinline__ void add(float m_s, float l_s, f32x4 v_s) {
+    const float gm = fmaxf(m, m_s);
+    const float r1 = fast_exp2(m - gm);
+    const float r2 = fast_exp2(m_s - gm);
+    l = l * r1 + l_s * r2;
+    v = v * r1 + v_s * r2;
+    m = gm;
   }
+};
+
+// Item (query g, outputs e .. e + 3) of a partial at `off` (bytes, the same
+// for all lanes) of the partials, with device-scope stores.  Row g of a
+// partial: D outputs, then (max, sum, 0, 0).
+template <int D>
+__device__ __forceinline__ void store_partial(Rsrc16 prs, int off, int g, int e, float m, float l, f32x4 v) {
+  using S = AttnShape<D>;
+  store16_sc1(prs, (g * S::kRow + e) * 4, off, v);
+  if (e == 0) store16_sc1(prs, (g * S::kRow + D) * 4, off, f32x4{m, l, 0.f, 0.f});
+}
+
+// A unit done by several workgroups: this one waits until its partials'
+// stores are acknowledged, then counts itself on the unit's counter.  True
+// for the one that counts last of `parts`: the others' stores are complete
+// before their counts, so it can read them without waiting, and it resets
+// the counter for the next launch.
+__device__ __forceinline__ bool count_part(const AttnArgs& a, int unit, int parts, int* s_last, int tid) {
   // Device-scope write-throughs: once this thread's are acknowledged they are
   // visible to every workgroup.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -486,19 +482,18 @@ __device__ __forceinline__ bool count_partial(const AttnArgs& a, const MergeShar
 }
 
 // Merge of a unit's `parts` partials in index order (so the result does not
-// depend on arrival order); part i is at place_of(i) (bytes), part `own` is
-// this workgroup's, taken from LDS.  The others' words of kGroupS parts are
-// requested at once.
-template <int DT, int D, typename PlaceOf>
-__device__ __forceinline__ void merge_partials(const AttnArgs& a, const MergeShared<D>& sh, Rsrc16 prs, int row,
-                                               int head0, int gcount, int parts, int own, int tid, PlaceOf place_of) {
+// depend on arrival order); part i is at place_of(i) (bytes, the same for all lanes), part `own` is
+// this workgroup's, from own_item(item, max, sum) (none if negative).  The
+// others' words of kGroupS parts are requested at once.
+template <int DT, int D, typename PlaceOf, typename OwnItem>
+__device__ __forceinline__ void merge_partials(const AttnArgs& a, Rsrc16 prs, int row, int head0, int gcount,
+                                               int parts, int own, int tid, PlaceOf place_of, OwnItem own_item) {
   using S = AttnShape<D>;
   constexpr int kChunks = D / 4;
   for (int item = tid; item < gcount * kChunks; item += kThreadsA) {
     const int g = item / kChunks;
     const int e = 4 * (item % kChunks);
-    float run_m = -INFINITY, run_l = 0.f;
-    f32x4 run = f32x4{0.f, 0.f, 0.f, 0.f};
+    Merged run;
     for (int s0 = 0; s0 < parts; s0 += kGroupS) {
       const int cnt = min(kGroupS, parts - s0);
       f32x4 pv[kGroupS];
@@ -507,9 +502,9 @@ __device__ __forceinline__ void merge_partials(const AttnArgs& a, const MergeSha
       for (int u = 0; u < kGroupS; ++u) {
         const int sp = s0 + u;
         if (u < cnt && sp != own) {
-          const uint32_t row_off = place_of(sp) + static_cast<uint32_t>(g * S::kRow * 4);
-          pv[u] = load16_sc1(prs, row_off + e * 4);
-          pml[u] = load8_sc1(prs, row_off + D * 4);
+          const int at = place_of(sp);
+          pv[u] = load16_sc1(prs, (g * S::kRow + e) * 4, at);
+          pml[u] = load8_sc1(prs, (g * S::kRow + D) * 4, at);
         }
       }
 #pragma unroll
@@ -519,21 +514,16 @@ __device__ __forceinline__ void merge_partials(const AttnArgs& a, const MergeSha
         float m_s, l_s;
         f32x4 a_s;
         if (sp == own) {
-          a_s = span_item<D>(sh, g, e, m_s, l_s);
+          a_s = own_item(item, m_s, l_s);
         } else {
           m_s = pml[u][0];
           l_s = pml[u][1];
           a_s = pv[u];
         }
-        const float gm = fmaxf(run_m, m_s);
-        const float r1 = fast_exp2(run_m - gm);
-        const float r2 = fast_exp2(m_s - gm);
-        run_l = run_l * r1 + l_s * r2;
-        run = run * r1 + a_s * r2;
-        run_m = gm;
+        run.add(m_s, l_s, a_s);
       }
     }
-    store_out<DT>(a, row, head0 + g, e, run, 1.f / run_l);
+    store_out<DT>(a, row, head0 + g, e, run.v, 1.f / run.l);
   }
 }
 
@@ -767,7 +757,7 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   }
 
   if (qb == 0 && split == pos / S::kSpan) write_token<D>(a, work_base, pos, kin, vin, threadIdx.x);
-  waves_to_lds<D>(sh, run, wave, quad, col);
+  waves_to_lds<D>(sh, run, wave, quad, col, gcount);
   lds_barrier();
   if (active == 1) {
     write_outputs<DT, D>(a, sh, row, head0, gcount, threadIdx.x);
@@ -780,10 +770,16 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
   constexpr int kPartBytes = kGroupQ * S::kRow * 4;
   const Rsrc16 prs = make_rsrc16(a.partials + static_cast<int64_t>(unit) * a.splits * kGroupQ * S::kRow,
                                  static_cast<int64_t>(a.splits) * kPartBytes);
-  if (count_partial<D>(a, sh, prs, static_cast<uint32_t>(split * kPartBytes), gcount, unit, active, &s_last,
-                       threadIdx.x)) {
-    merge_partials<DT, D>(a, sh, prs, row, head0, gcount, active, split, threadIdx.x,
-                          [](int sp) { return static_cast<uint32_t>(sp * kPartBytes); });
+  for (int item = threadIdx.x; item < gcount * (D / 4); item += kThreadsA) {
+    const int g = item / (D / 4), e = 4 * (item % (D / 4));
+    float mx, total_l;
+    const f32x4 v = span_item<D>(sh, g, e, mx, total_l);
+    store_partial<D>(prs, split * kPartBytes, g, e, mx, total_l, v);
+  }
+  if (count_part(a, unit, active, &s_last, threadIdx.x)) {
+    merge_partials<DT, D>(
+        a, prs, row, head0, gcount, active, split, threadIdx.x, [](int sp) { return sp * kPartBytes; },
+        [&](int item, float& m, float& l) { return span_item<D>(sh, item / (D / 4), 4 * (item % (D / 4)), m, l); });
   }
   finish();
 }
@@ -793,45 +789,48 @@ __global__ __launch_bounds__(kThreadsA, 2) void draft_attention_kernel(AttnArgs 
 // workgroup per span lost to it on large batches: every workgroup pays its
 // own ramp, wave merge and partial, rows' empty spans are launched too, and
 // the last round of workgroups is partly empty.
-//   - The tokens of every (row, KV head, query block) unit are cut into steps
-//     of 128 (32 per wave); the steps of all units are numbered unit by unit
-//     (a prefix sum over the rows' positions, in LDS), and each resident
-//     workgroup takes one contiguous range, so all end together whatever the
-//     rows' lengths.
-//   - Within a unit a wave requests the next step's K as soon as the score
+//   - The spans of every (row, KV head, query block) unit are numbered unit
+//     by unit (a prefix sum over the rows' positions, in LDS), and each
+//     resident workgroup takes one contiguous range, so all end together
+//     whatever the rows' lengths.
+//   - Within a unit a wave requests the next 32 tokens' K as soon as the score
 //     MFMAs have read the current K, and the next V after the output MFMAs.
+//   - Each span is computed and merged over the waves as the one-shot kernel
+//     does it, and the spans join in index order (Merged): a row's bits are
+//     the same in either kernel, whatever the other rows are and wherever the
+//     ranges end.
 //   - A unit inside one range is finished in place.  A unit cut by range
-//     ends is merged by the workgroup that counts last on it, partials in
-//     range order (the result does not depend on arrival).  A range has at
-//     most two cut units, its first and its last: two partial slots.
-// Fewer, longer ranges won: every unit boundary costs a merge and a cold
-// start, and 4 waves x 16 KB in flight per CU already fill the memory queue.
+//     ends (a range has two such units at most) leaves its first range's sum
+//     and the later ranges' spans as partials, and the workgroup that counts
+//     last on it continues the sum.
 // us on 57 rows of 300-3970 tokens (64/8 heads x 128, fp16) / 64 rows of 1987
 // (32/4 x 128) / 16 rows of 1984-3990 (32/8 x 256) / 48 rows of 984-1990
-// (32/8 x 64); bandwidth of the last line 5.5, 6.1, 5.6 and 4.9 TB/s:
-//   one workgroup per span, cached half lines       184 / 63 / 130 / 43.5
-//   ranges, 1 workgroup per CU (2 at 64), the same  107 / 48 /  82 / 34.8
-//   whole lines, non-temporal, 2 (2, 3) per CU       94 / 46.5 / 71 / 32.8
-//   whole lines, non-temporal, 1 (1, 2) per CU, kept 98 / 42.8 / 70 / 30.2
-// With the cached reads: two steps in flight per wave 110 / 48.6 / 82 / 35.5;
-// the next unit's operands requested before the merge 105 / 54 / 82 / 34.9,
-// no gain for 35 more registers.
+// (32/8 x 64); bandwidth of the last line 5.6, 6.1, 5.3 and 4.4 TB/s:
+//   one workgroup per span, cached half lines             184 / 63 / 130 / 43.5
+//   cut at any 128 tokens, one partial per range (a row's
+//     rounding then depends on the other rows)            98 / 42.7 / 70 / 30.1
+//   whole spans, later ranges' spans stored one by one    97 / 43.4 / 79 / 34.5
+//   held in LDS and stored when the unit ends, kept       96 / 43.0 / 74 / 33.8
+// The stores are what the later ranges' spans cost (without them 90 / - / 71 /
+// 30.8; writes at about 1% of the read bytes).  2 workgroups per CU at
+// head_dim 64 (1: 39); 1 else, where 4 waves x 16 KB in flight per CU already
+// fill the memory queue.
 template <int D>
 struct StreamShape {
-  static constexpr int kStep = kWavesA * 2 * kTileT;            // tokens per step (32 per wave)
-  static constexpr int kPerCu = D == 64 ? 2 : 1;       // workgroups per CU
+  static constexpr int kPerCu = D == 64 ? 2 : 1;            // workgroups per CU
+  static constexpr int kHeld = (D == 64 ? 40 : 64) * 1024;  // LDS bytes of held span results
   // Spans above which the batch is streamed: about one round of one-shot
   // workgroups (4 per CU at head_dim 64, 2 at 128).  us, one-shot against
   // streamed, at 512 spans of head_dim 128: 16.6 / 17.2 (16 rows of 1987
-  // tokens), 14.4 / 17.2 (64 rows of 184-487); at 576: 21.0 / 20.4; at 768:
-  // 26.2 / 23.8 (1987 tokens), 18.9 / 13.8 (100-400).  Head_dim 64, 1024
-  // spans: 17.7 / 17.6 (32 x 1987), 14.6 / 16.2 (64 rows of 184-487).
-  // Head_dim 256, 256 spans 18.8 / 18.6, 512 spans 23.5 / 21.6.
-  static constexpr int kOneRound = D == 64 ? 1024 : (D == 128 ? 512 : 256);
+  // tokens), 14.4 / 17.2 (64 rows of 184-487); 576: 21.8 / 22.5; 768: 26.9 /
+  // 24.1 (1987 tokens), 22.7 / 17.9 (100-1987).  Head_dim 64, 1152 spans:
+  // 19.9 / 22.5 (36 x 1987); 1280: 18.9 / 18.3 (100-1987); 1536: 26.0 / 26.6
+  // (1987); 4096: 53.3 / 41.1 (1000-1987).  Head_dim 256, 320 spans: 21.5 /
+  // 20.7; 576: 28.5 / 27.7; 1024: 43.5 / 32.5.
+  static constexpr int kOneRound = D == 64 ? 1152 : (D == 128 ? 576 : 256);
 };
-constexpr int kMinSteps = 2;  // steps per workgroup, at least
 
-struct Steps {  // workgroup w < used takes steps [start(w), start(w + 1))
+struct Ranges {  // workgroup w < used takes spans [start(w), start(w + 1))
   int base, rem, used;
   __device__ __forceinline__ int start(int w) const { return w * base + min(w, rem); }
   __device__ __forceinline__ int owner(int x) const {
@@ -844,9 +843,12 @@ template <int DT, int D>
 __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_stream_kernel(AttnArgs a) {
   using S = AttnShape<D>;
   constexpr int J = S::kJ;
-  constexpr int kStep = StreamShape<D>::kStep;
+  constexpr int kPairs = S::kTiles / 2;  // 32-token pairs of a wave's quarter of a span
+  constexpr int kChunks = D / 4;
+  constexpr int kItems = kGroupQ * kChunks / kThreadsA;  // merge items per thread
   __shared__ MergeShared<D> sh;
-  __shared__ int s_prefix[kMaxRows + 1];  // steps of one unit of each row, exclusive prefix
+  __shared__ f32x4 s_held[StreamShape<D>::kHeld / sizeof(f32x4)];  // span results not stored yet
+  __shared__ int s_prefix[kMaxRows + 1];  // spans of one unit of each row, exclusive prefix
   __shared__ int s_pos[kMaxRows];
   __shared__ int s_slot[kMaxRows];
   __shared__ int s_scratch[4];
@@ -867,7 +869,7 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
     if (pos >= a.budget) pos = -1;
     s_pos[r] = max(pos, -1);
     s_slot[r] = slot;
-    return pos >= 0 ? (pos + kStep) / kStep : 0;
+    return pos >= 0 ? (pos + S::kSpan) / S::kSpan : 0;
   });
   // Every thread's reads of the positions and the epoch have landed (the
   // prefix's barriers waited for them): the workgroup's seen word may go out.
@@ -879,15 +881,15 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
   }
 
   const int total = __builtin_amdgcn_readfirstlane(s_prefix[a.rows]) * units_row;
-  Steps st;
-  st.used = min(static_cast<int>(gridDim.x), max(1, total / kMinSteps));
+  Ranges st;
+  st.used = min(static_cast<int>(gridDim.x), max(1, total));
   st.base = __builtin_amdgcn_readfirstlane(total / st.used);
   st.rem = total - st.base * st.used;
   const int w = blockIdx.x;
   const int first = w < st.used ? st.start(w) : 0;
   const int end = w < st.used ? st.start(w + 1) : 0;
 
-  // One unit: row, KV head, query block and its steps [s0, s0 + count).
+  // One unit: row, KV head, query block and its spans [s0, s0 + count).
   struct Unit {
     int row, kvh, qb, s0, count, pos;
     int64_t work;  // element offset of the working rows
@@ -903,7 +905,7 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
     u.row = __builtin_amdgcn_readfirstlane(lo);
     row_hint = u.row;
     u.pos = __builtin_amdgcn_readfirstlane(s_pos[u.row]);
-    u.count = (u.pos + kStep) / kStep;
+    u.count = (u.pos + S::kSpan) / S::kSpan;
     const int base = __builtin_amdgcn_readfirstlane(s_prefix[u.row]) * units_row;
     const int k = __builtin_amdgcn_readfirstlane((s - base) / u.count);
     u.s0 = base + k * u.count;
@@ -919,129 +921,213 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
     u.work = uniform64(u.work);
     return u;
   };
-  // This wave's 32 tokens of step s start at token_of(u, s).
-  auto token_of = [&](const Unit& u, int s) { return (s - u.s0) * kStep + wave * (kStep / kWavesA); };
+  // This wave's quarter of span s starts at token_of(u, s).
+  auto token_of = [&](const Unit& u, int s) { return (s - u.s0) * S::kSpan + wave * (S::kTiles * kTileT); };
   auto kin_of = [&](const Unit& u) { return static_cast<const uint16_t*>(a.k_in) + u.row * a.k_row + u.kvh * a.k_head; };
   auto vin_of = [&](const Unit& u) { return static_cast<const uint16_t*>(a.v_in) + u.row * a.v_row + u.kvh * a.v_head; };
-  // Loads of the 32 tokens from tb on: buffer loads from the unit's working
-  // rows (a scalar base, one lane offset, fixed steps).  Rows at or past the
-  // position come from the new token's input row instead (its scores past
-  // the position are masked): the unit's last waves choose per lane.
+  // Loads of the 32 tokens from tb on: buffer loads whose resource ends at the
+  // position, so rows from there on are zeros and cost nothing.  One path for
+  // every tile: with a branch here the compiler sees a path on which V was not
+  // requested after K, and its waits for K wait for V too.
   const int k_lane = (line_token(col, 0) * D + line_elem(quad, col, 0)) * 2;
   const int v_lane = (4 * quad * D + v_elem<J>(col)) * 2;
-  const int unit_bytes = a.budget * D * 2;
-  auto load_k = [&](KTiles<D>& T, const Unit& u, int token) {
-    const int tb = __builtin_amdgcn_readfirstlane(token);
-    const uint16_t* rows_k = static_cast<const uint16_t*>(a.work_k) + uniform64(u.work);
-    if (tb + 2 * kTileT <= u.pos) {  // wave-uniform
-      const Rsrc16 r = make_rsrc16(rows_k, unit_bytes);
+  auto tile_rows = [&](const void* work, const Unit& u, int t) {  // (made scalar: see unit_at)
+    const int bytes = __builtin_amdgcn_readfirstlane(min(max(u.pos - t, 0), kTileT) * D * 2);
+    return make_rsrc16(static_cast<const uint16_t*>(work) + uniform64(u.work + static_cast<int64_t>(t) * D), bytes);
+  };
+  auto load_k = [&](KTiles<D>& T, const Unit& u, int tb) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int at = (tb + h * kTileT) * D * 2;
+    for (int h = 0; h < 2; ++h) {
+      const Rsrc16 r = tile_rows(a.work_k, u, tb + h * kTileT);
 #pragma unroll
-        for (int i = 0; i < S::kSteps; ++i) {
-          T.k[h][i] = __builtin_amdgcn_raw_buffer_load_b128(r, k_lane + 16 * (i & 1) * D + 128 * (i >> 1), at,
-                                                            kPolicyNt);
-        }
-      }
-    } else {
-      const uint16_t* in = kin_of(u);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int i = 0; i < S::kSteps; ++i) {
-          const int t = tb + h * kTileT + line_token(col, i);
-          T.k[h][i] = load16((t >= u.pos ? in : rows_k + static_cast<int64_t>(t) * D) + line_elem(quad, col, i));
-        }
+      for (int i = 0; i < S::kSteps; ++i) {
+        T.k[h][i] = __builtin_amdgcn_raw_buffer_load_b128(r, k_lane + 16 * (i & 1) * D + 128 * (i >> 1), 0, kPolicyNt);
       }
     }
   };
-  auto load_v = [&](VTiles<D>& T, const Unit& u, int token) {
-    const int tb = __builtin_amdgcn_readfirstlane(token);
-    const uint16_t* rows_v = static_cast<const uint16_t*>(a.work_v) + uniform64(u.work);
-    if (tb + 2 * kTileT <= u.pos) {  // wave-uniform
-      const Rsrc16 rs = make_rsrc16(rows_v, unit_bytes);
+  auto load_v = [&](VTiles<D>& T, const Unit& u, int tb) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 2; ++h) {
+      const Rsrc16 r = tile_rows(a.work_v, u, tb + h * kTileT);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) load_words_buf<J>(rs, v_lane + r * D * 2, (tb + h * kTileT) * D * 2, T.v[h][r]);
+      for (int i = 0; i < 4; ++i) load_words_buf<J>(r, v_lane + i * D * 2, 0, T.v[h][i]);
+    }
+  };
+  // The position's row is the new token's input row: the lane's slices of it,
+  // loaded with the unit's queries, go into the tile that holds the position.
+  u32x4 kin_s[S::kSteps / 2];
+  uint32_t vin_s[J / 2];
+  auto fix_k = [&](KTiles<D>& T, int at) {  // at = position - first token of the pair
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < S::kSteps; ++i) {
+        if (h * kTileT + line_token(col, i) == at) T.k[h][i] = kin_s[i / 2];
       }
-    } else {
-      const uint16_t* in = vin_of(u);
+    }
+  };
+  auto fix_v = [&](VTiles<D>& T, int at) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = tb + h * kTileT + 4 * quad + r;
-          load_words<J>((t >= u.pos ? in : rows_v + static_cast<int64_t>(t) * D) + v_elem<J>(col), T.v[h][r]);
-        }
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int w = 0; w < J / 2; ++w) T.v[h][i][w] = h * kTileT + 4 * quad + i == at ? vin_s[w] : T.v[h][i][w];
       }
     }
   };
   u32x4 qv[S::kSteps];
-  auto load_q = [&](const Unit& u) {
+  auto load_q = [&](const Unit& u) {  // columns past the unit's queries hold its last one and are not read out
     const int g0 = u.qb * kGroupQ, gcount = min(kGroupQ, a.group - g0);
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + u.row * a.q_row +
                          (u.kvh * a.group + g0 + min(col, gcount - 1)) * a.q_head + 8 * quad;
 #pragma unroll
-    for (int i = 0; i < S::kSteps; ++i) {
-      const u32x4 v = load16(qp + 32 * i);
-      qv[i] = col < gcount ? v : u32x4{0, 0, 0, 0};
-    }
+    for (int i = 0; i < S::kSteps; ++i) qv[i] = load16(qp + 32 * i);
+#pragma unroll
+    for (int i = 0; i < S::kSteps; i += 2) kin_s[i / 2] = load16(kin_of(u) + line_elem(quad, col, i));
+    load_words<J>(vin_of(u) + v_elem<J>(col), vin_s);
   };
 
   constexpr int kPartBytes = kGroupQ * S::kRow * 4;
-  const Rsrc16 prs = make_rsrc16(a.partials, static_cast<int64_t>(gridDim.x) * 2 * kPartBytes);
   const float c = a.scale * kLog2e;
   for (int s = first; s < end;) {
     const Unit u = unit_at(s);
     const int unit_end = u.s0 + u.count;
-    const int stop = min(unit_end, end);  // this range's steps of the unit: [s, stop)
-    const bool whole = s == u.s0 && stop == unit_end;
+    const int stop = min(unit_end, end);  // this range's spans of the unit: [s, stop)
+    const bool head = __builtin_amdgcn_readfirstlane(s == u.s0 ? 1 : 0) != 0;
     const int n = u.pos + 1;
+    const int g0 = u.qb * kGroupQ, gcount = min(kGroupQ, a.group - g0);
+    const int head0 = u.kvh * a.group + g0;
+    const int unit = (u.row * a.hkv + u.kvh) * a.qblocks + u.qb;
+    const Rsrc16 prs = make_rsrc16(a.partials + static_cast<int64_t>(unit) * a.splits * kGroupQ * S::kRow,
+                                   static_cast<int64_t>(a.splits) * kPartBytes);
+    // The unit's first range merges its spans in sum.  A later range holds
+    // each span's result in LDS, every thread its own items, and stores them
+    // when the unit (or the room) ends: a store among the loads delays the
+    // span.
+    Merged sum[kItems];
+    const int entries = gcount * (kChunks + 1);  // per held span: the outputs, then each query's (max, sum)
+    const int room = (StreamShape<D>::kHeld / static_cast<int>(sizeof(f32x4))) / entries;
+    int held = 0, held_at = s - u.s0;  // spans held, the first one's index in the unit
+    auto store_held = [&]() {
+      for (int h = 0; h < held; ++h) {
+        const int place = __builtin_amdgcn_readfirstlane((held_at + h) * kPartBytes);
+        for (int item = threadIdx.x; item < gcount * kChunks; item += kThreadsA) {
+          const int g = item / kChunks, e = 4 * (item % kChunks);
+          const f32x4 ml = s_held[h * entries + gcount * kChunks + g];
+          store_partial<D>(prs, place, g, e, ml[0], ml[1], s_held[h * entries + item]);
+        }
+      }
+      held_at += held;
+      held = 0;
+    };
     KTiles<D> K;
     VTiles<D> V;
+    load_q(u);
+    load_k(K, u, token_of(u, s));
+    load_v(V, u, token_of(u, s));
     Running<D> run;
     run.clear();
-    load_q(u);
-    int tb = token_of(u, s);
-    load_k(K, u, tb);
-    load_v(V, u, tb);
-    for (;;) {
-      const bool more = ++s < stop;
+    int tb = token_of(u, s), p = 0;
+    // One pair; MORE: the next one's loads are issued on the way (on every
+    // path: see load_k).
+    auto pair = [&](auto more) {
+      constexpr bool MORE = decltype(more)::value;
+      const bool span_end = !MORE || p == kPairs - 1;
+      const int next = span_end ? token_of(u, s + 1) : tb + 2 * kTileT;
+      const int at = __builtin_amdgcn_readfirstlane(u.pos - tb);
+      const bool holds_pos = at >= 0 && at < 2 * kTileT;  // wave-uniform
       f32x4 sc[2];
+      if (holds_pos) fix_k(K, at);
       pair_scores<DT, D>(K, qv, sc);
       __builtin_amdgcn_sched_barrier(0);
-      if (more) load_k(K, u, tb + kStep);
+      if constexpr (MORE) load_k(K, u, next);
       __builtin_amdgcn_sched_barrier(0);
       if (tb < n) {
-        zero_past<D>(V, tb, u.pos, quad);
+        if (holds_pos) fix_v(V, at);
         pair_output<DT, D>(V, sc, run, tb, n, quad, c);
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (!more) break;
-      tb += kStep;
-      load_v(V, u, tb);
-    }
-    const int g0 = u.qb * kGroupQ, gcount = min(kGroupQ, a.group - g0);
-    const int head0 = u.kvh * a.group + g0;
-    if (u.qb == 0 && stop == unit_end) write_token<D>(a, u.work, u.pos, kin_of(u), vin_of(u), threadIdx.x);
-    waves_to_lds<D>(sh, run, wave, quad, col);
-    lds_barrier();
-    if (whole) {
-      write_outputs<DT, D>(a, sh, u.row, head0, gcount, threadIdx.x);
-    } else {
-      const int w0 = st.owner(u.s0);
-      const int parts = st.owner(unit_end - 1) - w0 + 1;
-      auto place_of = [&](int i) {  // slot 1 of a range that starts in an earlier unit, else slot 0
-        return static_cast<uint32_t>((2 * (w0 + i) + (st.start(w0 + i) < u.s0 ? 1 : 0)) * kPartBytes);
-      };
-      const int unit = (u.row * a.hkv + u.kvh) * a.qblocks + u.qb;
-      if (count_partial<D>(a, sh, prs, place_of(w - w0), gcount, unit, parts, &s_last, threadIdx.x)) {
-        merge_partials<DT, D>(a, sh, prs, u.row, head0, gcount, parts, w - w0, threadIdx.x, place_of);
+      if constexpr (MORE) load_v(V, u, next);
+      tb = next;
+      ++p;
+      if (!span_end) return;
+      lds_barrier();  // every wave has read the previous span's states
+      waves_to_lds<D>(sh, run, wave, quad, col, gcount);
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int item = threadIdx.x + i * kThreadsA;
+        if (item < gcount * kChunks) {
+          const int g = item / kChunks, e = 4 * (item % kChunks);
+          float mx, total_l;
+          const f32x4 v = span_item<D>(sh, g, e, mx, total_l);
+          if (head) {
+            sum[i].add(mx, total_l, v);
+          } else {
+            s_held[held * entries + item] = v;
+            if (e == 0) s_held[held * entries + gcount * kChunks + g] = f32x4{mx, total_l, 0.f, 0.f};
+          }
+        }
       }
+      if (!head && ++held == room) store_held();
+      run.clear();
+      ++s;
+      p = 0;
+    };
+    for (int left = (stop - s) * kPairs; left > 1; --left) pair(std::true_type{});
+    pair(std::false_type{});
+    if (u.qb == 0 && stop == unit_end) write_token<D>(a, u.work, u.pos, kin_of(u), vin_of(u), threadIdx.x);
+    if (head && stop == unit_end) {
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int item = threadIdx.x + i * kThreadsA;
+        if (item < gcount * kChunks) {
+          store_out<DT>(a, u.row, head0 + item / kChunks, 4 * (item % kChunks), sum[i].v, 1.f / sum[i].l);
+        }
+      }
+      continue;
     }
-    lds_barrier();  // the next unit's states overwrite these
+    // A unit cut by range ends: its first range's sum is the first part, the
+    // later ranges' spans the others.  The first range is mostly the last to
+    // end (it meets the unit at its end, the others at their start): it looks
+    // whether all others have counted before it stores anything.
+    const int w0 = st.owner(u.s0);
+    const int ranges = st.owner(unit_end - 1) - w0 + 1;
+    const int skip = __builtin_amdgcn_readfirstlane(st.start(w0 + 1) - u.s0 - 1);  // spans of the sum besides span 0
+    bool last = false;
+    if (head) {
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {  // (nothing is held in a first range)
+        const int item = threadIdx.x + i * kThreadsA;
+        if (item < gcount * kChunks) {
+          s_held[item] = sum[i].v;
+          if (item % kChunks == 0) s_held[gcount * kChunks + item / kChunks] = f32x4{sum[i].m, sum[i].l, 0.f, 0.f};
+        }
+      }
+      if (threadIdx.x == 0) {
+        s_last = coherent_load(a.counters + unit) == static_cast<uint32_t>(ranges - 1) ? 1 : 0;
+        if (s_last != 0) coherent_store(a.counters + unit, 0u);
+      }
+      lds_barrier();
+      last = __builtin_amdgcn_readfirstlane(s_last) != 0;
+      if (!last) held = 1;
+    }
+    if (!last) {
+      store_held();
+      last = count_part(a, unit, ranges, &s_last, threadIdx.x);
+    }
+    if (last) {
+      merge_partials<DT, D>(
+          a, prs, u.row, head0, gcount, u.count - skip, head ? 0 : -1, threadIdx.x,
+          [skip](int i) { return (i == 0 ? 0 : i + skip) * kPartBytes; },
+          [&](int item, float& m, float& l) {
+            const f32x4 ml = s_held[gcount * kChunks + item / kChunks];
+            m = ml[0];
+            l = ml[1];
+            return s_held[item];
+          });
+    }
   }
   if (blockIdx.x == gridDim.x - 1) publish(a, tag, gridDim.x);
 }
@@ -1049,12 +1135,10 @@ __global__ __launch_bounds__(kThreadsA, StreamShape<D>::kPerCu) void attention_s
 template <int DT, int D>
 int launch_attention(hipStream_t stream, const AttnArgs& a) {
   const int64_t spans = static_cast<int64_t>(a.rows) * a.hkv * a.qblocks * a.splits;
-  const int64_t steps = static_cast<int64_t>(a.rows) * a.hkv * a.qblocks *
-                        ((a.budget + StreamShape<D>::kStep - 1) / StreamShape<D>::kStep);
-  // (32-bit step numbers and byte offsets within a unit's rows.)
-  if (spans > StreamShape<D>::kOneRound && steps < (int64_t{1} << 30) && static_cast<int64_t>(a.budget) * D * 2 < INT32_MAX) {
-    // Two partial slots per workgroup, out of the workspace's one per span.
-    const int64_t grid = std::min<int64_t>(static_cast<int64_t>(StreamShape<D>::kPerCu) * device_cu_count(), spans / 2);
+  // (32-bit span numbers and byte offsets within a unit's rows.)
+  if (spans > StreamShape<D>::kOneRound && spans < (int64_t{1} << 30) && static_cast<int64_t>(a.budget) * D * 2 < INT32_MAX) {
+    // (One seen word per workgroup, out of the workspace's one per span.)
+    const int64_t grid = std::min<int64_t>(static_cast<int64_t>(StreamShape<D>::kPerCu) * device_cu_count(), spans);
     attention_stream_kernel<DT, D><<<static_cast<unsigned>(grid), kThreadsA, 0, stream>>>(a);
     return check_launch("ds_draft_attention");
   }
