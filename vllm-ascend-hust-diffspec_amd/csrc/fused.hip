@@ -40,11 +40,12 @@
 // Polling is the costly part of this design: every poll is a device-scope
 // request to one memory channel, and thousands of waves polling one line
 // slow every stream that shares the channel.  So each row's tagged plan has
-// lines of its own and polls sleep between tries.  The row selectors (at
-// most kSelectors, each on one row at a time) poll their rows' partials
-// whole: at most kSelectors rows of partials per round trip (8 KB for a
-// 16k-token row with 4 KV heads), and no round trip for a sentinel word
-// between the row's last partial and its selection.
+// lines of its own and polls sleep between tries.  The row selectors (8 for
+// long rows, up to one per 4 CUs for short ones, see selectors.h; each on one
+// row at a time) poll their rows' partials whole: one row of partials per
+// selector and round trip (8 KB for a 16k-token row with 4 KV heads), and no
+// round trip for a sentinel word between the row's last partial and its
+// selection.
 //
 // Forward progress does not depend on all workgroups being resident at once
 // (the launch is an ordinary one).  Workgroups are dispatched in index order
@@ -77,6 +78,7 @@
 #include "gather_body.h"
 #include "score_body.h"
 #include "select_body.h"
+#include "selectors.h"
 
 namespace ds355 {
 
@@ -102,26 +104,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-// Row selectors (fewer when the batch has fewer rows).  8 against 16, events
-// around each launch, two rounds: 16 rows of 4k-40k tokens 82.5-82.7 against
-// 82.8-83.4 us (other seeds 0.3-1.4 us faster), 16 x 40k 156.2-156.4
-// against 157.1-157.6 us, 64 rows equal or faster.  A selector's rows
-// complete tens of microseconds apart, and the freed slots score.  4
-// selectors: 0.5-0.9 us slower on the first draw, up to 1 us faster on
-// others; 2: 25-45% slower on ragged rows (selections queue).
-constexpr int kSelectors = 8;
-// Short rows complete together, and then the selections queue: a selector
-// takes about 5 us a row, in which the device streams about
-// kBytesPerSelection of keys.  So a batch whose score buffer holds few keys
-// gets enough selectors for its selections to take no longer than its
-// scoring, at most kMaxSelectors (row_selectors).  us with 8 / as many as rows
-// / this rule: 36 rows of 1.7k tokens (16/2 heads x 64) 48.6 / 27.6 / 27.7,
-// 11 rows of 469-1591 23.9 / 18.5 / 18.5, 16 rows of 1-2k (32/4 x 128) 32.8 /
-// 32.1 / 32.9; but 64 rows of 1-4k 122.3 / 126.6, 16 x 40k 147.5 / 150.5:
-// workgroups that only wait lengthen the scoring there.  (Counted from the
-// rows' own lengths on the device instead, every launch was 1-3 us slower.)
-constexpr int kMaxSelectors = 64;
-constexpr int64_t kBytesPerSelection = int64_t{27} << 20;
 // Without a supplied LSE: workgroups doing the KV groups' shares, below the
 // row selectors.  Measured on 16 rows of 4k-40k tokens (one step): 32 group
 // workgroups 96.6-98.3 us; 16 of them 101.9 us; 32 with the last group's
@@ -790,14 +772,6 @@ __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
   }
 }
 
-// Row selectors of a launch over `upper_units` scoring units at most (see
-// kMaxSelectors).
-int row_selectors(int rows, const score::ScoreArgs& s, int64_t upper_units) {
-  const int64_t bytes = std::max<int64_t>(1, upper_units * s.U * s.D * 2);
-  const int64_t want = std::min<int64_t>(rows * kBytesPerSelection / bytes, kMaxSelectors);
-  return std::min(rows, std::max(kSelectors, static_cast<int>(want)));
-}
-
 size_t plans_bytes(int rows) { return static_cast<size_t>(rows) * kPlanCols * sizeof(uint64_t); }
 int task_cap(int token_budget) { return (token_budget + kMinTaskPositions - 1) / kMinTaskPositions; }
 size_t state_bytes(int rows, int token_budget) {
@@ -934,7 +908,7 @@ int launch_fused_step(hipStream_t stream, const ds_step_desc* d, const RowSource
   f.task_cap = task_cap(d->token_budget);
   ws += state_bytes(d->batch_rows, d->token_budget);
   f.s.tagged = reinterpret_cast<uint64_t*>(ws);
-  f.selectors = row_selectors(d->batch_rows, f.s, upper_units);
+  f.selectors = row_selectors(d->batch_rows, upper_units * f.s.U * f.s.D * 2, device_cu_count());
   f.owner_spins = (d->flags & DS_STEP_SELECTORS_GATHER) != 0 ? 0u : kOwnerSpins;
   f.expire = (d->flags & DS_STEP_EXPIRE_WAITS) != 0 ? 1 : 0;
   f.status_out = status_out;
