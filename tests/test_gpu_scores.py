@@ -17,13 +17,13 @@ from helpers import O, assert_scores_close, default_scale, gen, lse_for, paged_k
 pytestmark = pytest.mark.gpu
 
 
-def _gpu_scores(query, key_cache, lse, table, lengths, chunk, scale, device, head_reduce="mean"):
+def _gpu_scores(query, key_cache, lse, table, lengths, chunk, scale, device, head_reduce="mean", width=None):
     from ds355.kernels import paged_chunk_attention_scores
 
     return paged_chunk_attention_scores(
         query.to(device), key_cache.to(device), None if lse is None else lse.to(device), table.to(device),
         torch.tensor(lengths, dtype=torch.int32, device=device),
-        chunk_size=chunk, max_seq_len=max(lengths), scale=scale, head_reduce=head_reduce,
+        chunk_size=chunk, max_seq_len=width or max(lengths), scale=scale, head_reduce=head_reduce,
     ).cpu()
 
 
@@ -129,24 +129,28 @@ def _page_dense(dense, block_size, pad):
 @pytest.mark.parametrize("block_size,pad", [(16, 0), (48, 8)])
 @pytest.mark.parametrize("mode", ["mean", "max", "free"])
 def test_whole_line_loads_give_the_bits_of_half_line_loads(cuda, head_dim, block_size, pad, mode):
-    # Blocks of whole 16-token groups read keys in 128-byte lines and exchange
-    # halves between lanes; other blocks (40 tokens) read the MFMA operands
-    # directly.  Same operands, same order: the same bits, at any row end
-    # within a group and with rows that are not line-aligned (pad).
+    # Blocks of whole 16-token groups in a launch that is large by its score
+    # buffer (110 MB of keys) read them in 128-byte lines and exchange halves
+    # between lanes; other blocks (40 tokens) and small launches read the MFMA
+    # operands directly.  Same operands, same order: the same bits, at any row
+    # end within a group and with rows that are not line-aligned (pad).
     g = gen(11)
     lengths = [1, 7, 8, 9, 15, 16, 17, 63, 65, 500]
     query = randn((len(lengths), 16, head_dim), torch.bfloat16, g)
     dense = [randn((n, 2, head_dim), torch.bfloat16, g) for n in lengths]
     lse = None if mode == "free" else torch.randn((len(lengths), 16), generator=g) + 4.0
+    wide = 110_000_000 // (len(lengths) * 2 * head_dim * 2)
     out = []
-    for bs, extra in ((block_size, pad), (40, 0)):
+    for bs, extra, width in ((block_size, pad, wide), (block_size, pad, None), (40, 0, wide)):
         keys, table = _page_dense(dense, bs, extra)
         device_keys = torch.empty((*keys.shape[:3], head_dim + extra), dtype=keys.dtype, device=cuda)[..., :head_dim]
         device_keys.copy_(keys)
         out.append(_gpu_scores(query, device_keys, lse, table, lengths, 64, head_dim ** -0.5, cuda,
-                               head_reduce="max" if mode == "max" else "mean"))
+                               head_reduce="max" if mode == "max" else "mean", width=width))
     assert torch.isfinite(out[0]).all()
-    assert torch.equal(out[0], out[1])
+    assert torch.equal(out[0], out[2])
+    chunks = out[1].shape[1]
+    assert torch.equal(out[0][:, :chunks], out[1]) and out[0][:, chunks:].count_nonzero() == 0
 
 
 @pytest.mark.parametrize("hkv,hq", [(1, 4), (2, 32), (4, 4), (8, 64), (16, 16), (3, 12)])

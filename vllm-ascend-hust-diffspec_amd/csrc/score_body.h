@@ -290,13 +290,15 @@ struct FinalShared {
 // FINAL (head mean, Hkv a power of two): units are dealt in groups (see
 // FinalShared), gw / tw are the workgroup's index and the grid, and the
 // workgroup writes the final scores itself.
-template <int DT, int STEPS, int KB, bool HMAX, int PAGE, bool TAGGED, bool LSEFREE = false, bool FINAL = false>
+// WHOLE: keys in whole lines where the shape allows it (LINES); the same bits.
+template <int DT, int STEPS, int KB, bool HMAX, int PAGE, bool TAGGED, bool LSEFREE = false, bool FINAL = false,
+          bool WHOLE = true>
 __device__ __forceinline__ void score_stream(const ScoreArgs& a, const int* s_prefix, const int* s_len,
                                              const int* s_qrow, int total, int gw, int tw, uint32_t tag,
                                              FinalShared* fin = nullptr) {
   constexpr bool UNIFORM_PAGE = PAGE != PAGE_LANE;
   constexpr bool POW2 = PAGE == PAGE_POW2;
-  constexpr bool LINES = UNIFORM_PAGE && STEPS % 2 == 0;  // whole-line key loads (swap_lines)
+  constexpr bool LINES = WHOLE && UNIFORM_PAGE && STEPS % 2 == 0;  // whole-line key loads (swap_lines)
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;   // A row (query head in group) / B column (token in group)
   const int kgrp = lane >> 4;  // 8-element k slice of the 32-wide MFMA step

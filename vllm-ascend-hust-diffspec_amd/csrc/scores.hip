@@ -51,7 +51,7 @@ using namespace score;
 // OUT = what the pass writes: per-KV-head partials, the mass words (no LSE
 // supplied) or final scores.
 enum { OUT_PARTIAL, OUT_MASS, OUT_FINAL };
-template <int DT, int STEPS, int KB, int WGS, bool HMAX, int PAGE, int OUT>
+template <int DT, int STEPS, int KB, int WGS, bool HMAX, int PAGE, int OUT, bool WHOLE>
 __global__ __launch_bounds__(kThreads, WGS) void chunk_score_kernel(ScoreArgs a) {
   constexpr bool FINAL = OUT == OUT_FINAL;
   __shared__ int s_prefix[kMaxRows + 1];
@@ -71,12 +71,12 @@ __global__ __launch_bounds__(kThreads, WGS) void chunk_score_kernel(ScoreArgs a)
   const int total = s_prefix[a.batch];
   if constexpr (FINAL) {
     __shared__ FinalShared s_final;
-    score_stream<DT, STEPS, KB, false, PAGE, false, false, true>(a, s_prefix, s_len, s_qrow, total, blockIdx.x,
+    score_stream<DT, STEPS, KB, false, PAGE, false, false, true, WHOLE>(a, s_prefix, s_len, s_qrow, total, blockIdx.x,
                                                                  gridDim.x, 0u, &s_final);
   } else {
     const int gw = uniform(blockIdx.x * kWaves + (threadIdx.x >> 6));
-    score_stream<DT, STEPS, KB, HMAX, PAGE, false, OUT == OUT_MASS>(a, s_prefix, s_len, s_qrow, total, gw,
-                                                                    gridDim.x * kWaves, 0u);
+    score_stream<DT, STEPS, KB, HMAX, PAGE, false, OUT == OUT_MASS, false, WHOLE>(a, s_prefix, s_len, s_qrow, total,
+                                                                                  gw, gridDim.x * kWaves, 0u);
   }
 
   if (a.write_tail) {
@@ -211,8 +211,25 @@ __global__ __launch_bounds__(kThreads) void lse_finalize_kernel(const uint64_t* 
   }
 }
 
+// Key bytes (of the score buffer's width) from which a launch reads keys in
+// whole lines.  A small one is bound by its waves' latency: the exchange of
+// halves and the longer way of a non-temporal load come on top, and the bytes
+// saved don't matter; the head max, with a wave per span walking all heads,
+// stays so the longest.  us in half lines, cached / whole lines, 30 inputs in
+// turn.  Mean with a LSE, a step's chain: 1 row of 1000 tokens (32/4 x 128)
+// 17.3 / 18.1, 1 x 8000 x 64 17.5 / 18.2, 1 x 8000 x 128 (8.2 MB) 19.4 / 18.7,
+// 1 x 30000 x 64 21.9 / 20.5; without one: 1 x 8000 x 64 13.1 / 13.7, 1 x
+// 8000 (32/8 x 64) 25.7 / 24.9.  Final scores: 1 x 8000 x 128 6.75 / 7.46,
+// (32/8 x 64) 8.5 / 9.2, 1 x 30000 x 64 (15 MB) 8.5 / 8.3, 1 x 8000 x 256 10.0 /
+// 9.2.  Head max: 1 x 300 (32/4 x 128) 14.4 / 15.6, 1 x 8192 15.1 / 16.6, 4 x
+// 4-9k (32/8 x 128, 74 MB) 27.1 / 27.8, 8 x 4-16k (32/4 x 128, 131 MB) 29.2 /
+// 27.9.
+constexpr int64_t kWholeMean = int64_t{7} << 20;
+constexpr int64_t kWholeFinal = int64_t{12} << 20;
+constexpr int64_t kWholeMax = int64_t{96} << 20;
+
 template <int DT, int STEPS, bool HMAX, int OUT>
-void launch_kb(hipStream_t stream, const ScoreArgs& a, int64_t upper_blocks, int page_mode) {
+void launch_kb(hipStream_t stream, const ScoreArgs& a, int64_t upper_blocks, int page_mode, bool whole) {
   // Batch shape: about 4 KB of keys per wave and batch at three workgroups
   // per CU.  At head_dim 128 one 16-token group (4 KB) beat two (8 KB) by
   // 1.3 us on 16 rows of 4k-40k tokens and 0.4-0.7 us on 16 x 40k and
@@ -231,26 +248,32 @@ void launch_kb(hipStream_t stream, const ScoreArgs& a, int64_t upper_blocks, int
   constexpr int WGS = narrow ? 3 : 2;
   const int64_t cap = static_cast<int64_t>(device_cu_count()) * WGS;
   const int grid = static_cast<int>(std::max<int64_t>(1, std::min(upper_blocks, cap)));
-  if (page_mode == PAGE_POW2) {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_POW2, OUT><<<grid, kThreads, 0, stream>>>(a);
-  } else if (page_mode == PAGE_UNIFORM) {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_UNIFORM, OUT><<<grid, kThreads, 0, stream>>>(a);
-  } else {
-    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, PAGE_LANE, OUT><<<grid, kThreads, 0, stream>>>(a);
-  }
+  auto launch = [&](auto page, auto lines) {
+    chunk_score_kernel<DT, STEPS, KB, WGS, HMAX, decltype(page)::value, OUT, decltype(lines)::value>
+        <<<grid, kThreads, 0, stream>>>(a);
+  };
+  auto launch_page = [&](auto page) {
+    if constexpr (STEPS % 2 == 0) {
+      if (whole) return launch(page, std::true_type{});
+    }
+    launch(page, std::false_type{});
+  };
+  if (page_mode == PAGE_POW2) launch_page(std::integral_constant<int, PAGE_POW2>{});
+  else if (page_mode == PAGE_UNIFORM) launch_page(std::integral_constant<int, PAGE_UNIFORM>{});
+  else launch(std::integral_constant<int, PAGE_LANE>{}, std::false_type{});
 }
 
 template <int DT, bool HMAX, int OUT>
-void launch_steps(hipStream_t stream, const ScoreArgs& a, int64_t grid, int page_mode) {
+void launch_steps(hipStream_t stream, const ScoreArgs& a, int64_t grid, int page_mode, bool whole) {
   switch (a.D / 32) {
-    case 1: launch_kb<DT, 1, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 2: launch_kb<DT, 2, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 3: launch_kb<DT, 3, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 4: launch_kb<DT, 4, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 5: launch_kb<DT, 5, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 6: launch_kb<DT, 6, HMAX, OUT>(stream, a, grid, page_mode); break;
-    case 7: launch_kb<DT, 7, HMAX, OUT>(stream, a, grid, page_mode); break;
-    default: launch_kb<DT, 8, HMAX, OUT>(stream, a, grid, page_mode); break;
+    case 1: launch_kb<DT, 1, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 2: launch_kb<DT, 2, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 3: launch_kb<DT, 3, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 4: launch_kb<DT, 4, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 5: launch_kb<DT, 5, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 6: launch_kb<DT, 6, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    case 7: launch_kb<DT, 7, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
+    default: launch_kb<DT, 8, HMAX, OUT>(stream, a, grid, page_mode, whole); break;
   }
 }
 
@@ -396,16 +419,18 @@ int launch_chunk_scores(hipStream_t stream, int dtype, const void* query, int64_
   // Groups of units for final scores (FinalShared): kWaves units, or one span's Hkv.
   const int group = final_out ? std::max(kWaves, num_kv_heads) : kWaves;
   const int64_t upper_blocks = (upper_units + group - 1) / group;
+  const int64_t key_bytes = upper_units * a.U * head_dim * 2 * (hmax ? num_kv_heads : 1);
+  const bool whole = key_bytes >= (hmax ? kWholeMax : (final_out ? kWholeFinal : kWholeMean));
   if (dtype == DS_BF16) {
-    if (hmax) launch_steps<DS_BF16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
-    else if (lse_free) launch_steps<DS_BF16, false, OUT_MASS>(stream, a, upper_blocks, page_mode);
-    else if (final_out) launch_steps<DS_BF16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode);
-    else launch_steps<DS_BF16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
+    if (hmax) launch_steps<DS_BF16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode, whole);
+    else if (lse_free) launch_steps<DS_BF16, false, OUT_MASS>(stream, a, upper_blocks, page_mode, whole);
+    else if (final_out) launch_steps<DS_BF16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode, whole);
+    else launch_steps<DS_BF16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode, whole);
   } else {
-    if (hmax) launch_steps<DS_FP16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
-    else if (lse_free) launch_steps<DS_FP16, false, OUT_MASS>(stream, a, upper_blocks, page_mode);
-    else if (final_out) launch_steps<DS_FP16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode);
-    else launch_steps<DS_FP16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode);
+    if (hmax) launch_steps<DS_FP16, true, OUT_PARTIAL>(stream, a, upper_blocks, page_mode, whole);
+    else if (lse_free) launch_steps<DS_FP16, false, OUT_MASS>(stream, a, upper_blocks, page_mode, whole);
+    else if (final_out) launch_steps<DS_FP16, false, OUT_FINAL>(stream, a, upper_blocks, page_mode, whole);
+    else launch_steps<DS_FP16, false, OUT_PARTIAL>(stream, a, upper_blocks, page_mode, whole);
   }
   int rc2 = check_launch("ds_chunk_scores");
   if (rc2 != DS_OK || !lse_free) return rc2;
