@@ -119,13 +119,14 @@ def test_gather_dtypes_and_layouts(cuda, dtype, neox, rotary_dim):
 @pytest.mark.parametrize("dtype,dim,rotary_dim,neox", [
     (torch.bfloat16, 64, 64, True), (torch.bfloat16, 64, 32, True), (torch.float16, 64, 32, False),
     (torch.float16, 64, 64, True), (torch.float32, 32, 16, False), (torch.float32, 32, 32, True)])
-@pytest.mark.parametrize("heads", [1, 5, 8])
-def test_gather_rows_of_one_line(cuda, dtype, dim, rotary_dim, neox, heads):
-    """Rows of 128 bytes, moved in whole lines by pairs of lanes: histories that end inside and
-    beside a task's 16 positions, heads in one and several groups."""
+@pytest.mark.parametrize("heads,rows", [(1, 13), (5, 13), (8, 13), (1, 12), (4, 5)])
+def test_gather_rows_of_one_line(cuda, dtype, dim, rotary_dim, neox, heads, rows):
+    """Rows of 128 bytes, moved in whole lines by pairs of lanes where there are 384 tasks (13 rows
+    of 30) and each by its own lanes where there are fewer: histories that end inside and beside a
+    task's 16 positions, heads in one and several groups."""
     chunk, token_budget, lmax = 32, 512, 900
     g = gen(9)
-    ends = [1, 2, 3, 4, 7, 15, 16, 17, 18, 31, 33, 480, 899]
+    ends = [899, 480, 1, 16, 33, 2, 3, 4, 7, 15, 17, 18, 31][:rows]
     slots = list(reversed(range(len(ends))))
     budget = O.history_budget(token_budget, 4, chunk)
     plans = []

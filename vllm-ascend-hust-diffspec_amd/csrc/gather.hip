@@ -36,7 +36,7 @@ using namespace gather;
 // one slot's raw cache ([max_model_len, H, D], below 2 GiB: checked on the
 // host) and one slot's working cache ([H, budget, D]); a lane with nothing
 // to move uses an out-of-range offset.
-template <int DT, bool NEOX, int HG>
+template <int DT, bool NEOX, int HG, bool LINES>
 __global__ __launch_bounds__(kThreads) void gather_wave_kernel(GatherArgs a) {
   __shared__ int s_prefix[kMaxRows + 1];
   __shared__ int s_scratch[4];
@@ -67,8 +67,8 @@ __global__ __launch_bounds__(kThreads) void gather_wave_kernel(GatherArgs a) {
     const int64_t tail_start = scalar_load(prow + 2);
     const int64_t prefix_len = scalar_load(prow + 3);
     const int64_t drop = scalar_load(prow + 4);
-    gather_task<DT, NEOX, HG, kLoadCached, true>(a, L, p0, slot, len, tail_start, prefix_len, drop, h0, min(h0 + HG, a.heads),
-                              [&](int64_t c) { return prow[5 + c]; });
+    gather_task<DT, NEOX, HG, kLoadCached, LINES>(a, L, p0, slot, len, tail_start, prefix_len, drop, h0,
+                                                  min(h0 + HG, a.heads), [&](int64_t c) { return prow[5 + c]; });
   }
 }
 
@@ -311,22 +311,31 @@ bool vector_path(GatherArgs& a, bool neox) {
   return vec;
 }
 
+// Tasks from which rows of one line are moved whole: fewer wait on latency,
+// to which the swaps add.  us without / with, head_dim 64, 124 tasks per row
+// and 4 heads: 1 x 4 heads 5.5 / 6.1, 1 x 8 and 2 x 4 (248 tasks) 5.95 / 6.35
+// and 6.1 / 6.4, 2 x 8 and 4 x 4 (496) 7.9 / 7.8 and 8.15 / 7.9, 8 x 8 18.3 / 16.8.
+constexpr int64_t kLineTasks = 384;
+
+template <int DT, bool NEOX, bool LINES>
+int launch_heads(hipStream_t stream, const GatherArgs& a, int64_t tasks) {
+  if (a.heads >= 4) return launch_wave<gather_wave_kernel<DT, NEOX, 4, LINES>>(stream, a, tasks);
+  if (a.heads >= 2) return launch_wave<gather_wave_kernel<DT, NEOX, 2, LINES>>(stream, a, tasks);
+  return launch_wave<gather_wave_kernel<DT, NEOX, 1, LINES>>(stream, a, tasks);
+}
+
 template <int DT>
 int launch_gather(hipStream_t stream, const GatherArgs& a, bool neox, bool vec, int grid) {
   if (vec) {
     const int ppw = 64 / a.lanes_per_row;
     const int hg = a.heads >= 4 ? 4 : (a.heads >= 2 ? 2 : 1);
     const int64_t tasks = static_cast<int64_t>(a.rows) * ((a.pos_limit + ppw - 1) / ppw) * ((a.heads + hg - 1) / hg);
-    if (a.heads >= 4) {
-      if (neox) return launch_wave<gather_wave_kernel<DT, true, 4>>(stream, a, tasks);
-      return launch_wave<gather_wave_kernel<DT, false, 4>>(stream, a, tasks);
+    if (a.lanes_per_row == 4 && tasks >= kLineTasks) {
+      if (neox) return launch_heads<DT, true, true>(stream, a, tasks);
+      return launch_heads<DT, false, true>(stream, a, tasks);
     }
-    if (a.heads >= 2) {
-      if (neox) return launch_wave<gather_wave_kernel<DT, true, 2>>(stream, a, tasks);
-      return launch_wave<gather_wave_kernel<DT, false, 2>>(stream, a, tasks);
-    }
-    if (neox) return launch_wave<gather_wave_kernel<DT, true, 1>>(stream, a, tasks);
-    return launch_wave<gather_wave_kernel<DT, false, 1>>(stream, a, tasks);
+    if (neox) return launch_heads<DT, true, false>(stream, a, tasks);
+    return launch_heads<DT, false, false>(stream, a, tasks);
   }
   gather_scalar_kernel<DT><<<grid, kThreads, 0, stream>>>(a, neox ? 1 : 0);
   return check_launch("ds_rebuild_compact_kv");
