@@ -656,6 +656,14 @@ __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
   // draft's, is 64 (the code for them costs 1.7 us of 108 on 16 rows without
   // an LSE at head_dim 128, which never runs it).
   constexpr bool LINES = STEPS == 2;
+  // Keys in whole lines, but for head_dim 64 with a LSE, where the exchange of
+  // halves costs more than the lines save.  us in half lines / whole lines at
+  // head_dim 64: 8 rows of 4-9k tokens (32/4 heads) 37.5 / 41.2, 17 + 17 of
+  // 23-35k (64/8) 158.8 / 162, 16 x 4-40k (32/8) 107.2 / 110.2, 64 x 2-20k
+  // (32/4) 125.5 / 127.3, 16 x 1-3k (32/8) 42.1 / 41.6; without a LSE 12 x 4-9k
+  // (32/8) 76.3 / 70.9, 16 x 20-40k 180 / 184.  At 128: 8 x 4-9k 44.9 / 42.9, 16 x
+  // 4-16k 59.0 / 55.6.
+  constexpr bool WHOLE = STEPS != 2 || LSEFREE;
   constexpr int KB = STEPS <= 2 ? 2 : 1;  // chunk_score_kernel's batch shape (4 KB) for head_dim <= 128
   __shared__ union {
     select::SelectShared<kFusedKeys> sel;
@@ -728,8 +736,8 @@ __global__ __launch_bounds__(kThreads, 3) void fused_step_kernel(FusedArgs f) {
     const int gw = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * kWaves +
                                                   static_cast<int>(threadIdx.x >> 6));
     const int tw = first_selector * kWaves;
-    score::score_stream<DT, STEPS, KB, false, PAGE, true, LSEFREE>(sa, w.unit_prefix, w.len, w.qrow,
-                                                                   w.unit_prefix[rows], gw, tw, tag);
+    score::score_stream<DT, STEPS, KB, false, PAGE, true, LSEFREE, false, WHOLE>(
+        sa, w.unit_prefix, w.len, w.qrow, w.unit_prefix[rows], gw, tw, tag);
     gather_owned<DT, NEOX, LINES>(f, s_task_prefix, s_slot, gw, tw, tag);
   }
 
