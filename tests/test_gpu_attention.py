@@ -440,3 +440,91 @@ def test_a_row_has_the_same_bits_in_any_batch(cuda, rows, hq, hkv, dim, budget, 
         assert not streamed
         _same_bits(alone[0], whole[r])
     assert attention.attention_status(dev.ws) == 0
+
+
+def test_streamed_and_one_shot_launches_share_a_workspace(cuda):
+    """One workspace, launches of both kernels in turn (their "seen" words and partials lie
+    elsewhere, the unit counters and the epoch are the same ones): each step has the oracle's
+    outputs, caches and lengths, its own epoch and a clear status."""
+    from ds355 import attention
+
+    case = Case(77, 30, 4, 32, 128, 2048)
+    for s in range(30):
+        case.fill(s, [0, 40, 255, 256, 700, 1500, 2030][s % 7] + s // 7)
+    dev = Device(case, cuda, 28)
+    plan = [(range(28), True), ([3, 17, 4], False), (range(29, 4, -1), True), ([9], False), (range(0, 30, 2), False),
+            (range(2, 30), True)]
+    for n, (slots, expect) in enumerate(plan, 1):
+        slots = list(slots)
+        _step(case, dev, cuda, slots, None, len(slots) + 1, 0.09)
+        assert attention.attention_epoch(dev.ws) == n
+        assert _launched_streamed(dev.ws, len(slots), 4, 8, 128, 2048, n) == expect
+
+
+@pytest.mark.parametrize("rows", [3, 40])
+@pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+def test_strided_rows_and_heads(cuda, rows, dim, dtype):
+    """Queries, keys and values that are parts of one packed buffer and an output with spare
+    elements give the bits of contiguous ones, in the one-shot and the streamed kernel."""
+    from ds355 import attention
+
+    hq, hkv, budget = 16, 4, 2048
+    case = Case(rows + dim, rows, hkv, hq, dim, budget, dtype)
+    lengths = [(331 * r + 7) % (budget - 1) for r in range(rows)]
+    for s, n in enumerate(lengths):
+        case.fill(s, n)
+    q, k, v = (t.to(cuda) for t in case.inputs(rows))
+    packed = torch.full((rows, hq + 2 * hkv + 1, dim + 8), float("nan"), dtype=dtype, device=cuda)[..., :dim]
+    packed[:, :hq], packed[:, hq: hq + hkv], packed[:, hq + hkv: hq + 2 * hkv] = q, k, v
+    wide = torch.full((rows, hq + 3, dim + 16), float("nan"), dtype=dtype, device=cuda)
+    results = []
+    for args, out in (((q, k, v), torch.empty_like(q)),
+                      ((packed[:, :hq], packed[:, hq: hq + hkv], packed[:, hq + hkv: hq + 2 * hkv]),
+                       wide[:, 1: hq + 1, 8: dim + 8])):
+        dev = Device(case, cuda, rows)
+        attention.draft_linear_attention(*args, out, dev.k, dev.v, dev.lens, list(range(rows)), None,
+                                         scale=dim ** -0.5, workspace=dev.ws)
+        results.append((out.cpu(), dev.k.cpu(), dev.v.cpu(), dev.lens.cpu()))
+        assert _launched_streamed(dev.ws, rows, hkv, hq // hkv, dim, budget, 1) == (rows == 40)
+    for a, b in zip(*results):
+        _same_bits(a, b)
+    outside = wide.cpu()
+    outside[:, 1: hq + 1, 8: dim + 8] = float("nan")
+    assert outside.isnan().all()
+
+
+def test_streamed_launch_replayed_from_a_graph(cuda):
+    """A captured streamed launch, replayed with other inputs and the eager launch between the
+    replays, gives the eager launch's bits every time."""
+    from ds355 import attention
+
+    rows, hq, hkv, dim, budget = 28, 32, 4, 128, 2048
+    case = Case(5, rows, hkv, hq, dim, budget)
+    for s in range(rows):
+        case.fill(s, (211 * s + 250) % (budget - 6))
+    slots = torch.tensor([(5 * r + 2) % rows for r in range(rows)], dtype=torch.int32, device=cuda)
+    q, k, v = (t.to(cuda) for t in case.inputs(rows + 2))
+    graphed, eager, warm = (Device(case, cuda, rows) for _ in range(3))
+
+    def launch(dev):
+        out = torch.full_like(q, float("nan"))
+        attention.draft_linear_attention(q, k, v, out, dev.k, dev.v, dev.lens, slots, None, scale=dim ** -0.5,
+                                         workspace=dev.ws)
+        return out
+
+    launch(warm)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = launch(graphed)
+    for step in range(1, 5):
+        for buffer, fresh in zip((q, k, v), case.inputs(rows + 2)):
+            buffer.copy_(fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        expected = launch(eager)
+        _same_bits(out.cpu(), expected.cpu())
+        for a, b in ((graphed.k, eager.k), (graphed.v, eager.v), (graphed.lens, eager.lens)):
+            _same_bits(a.cpu(), b.cpu())
+        assert attention.attention_epoch(graphed.ws) == step and attention.attention_status(graphed.ws) == 0
+        assert _launched_streamed(graphed.ws, rows, hkv, hq // hkv, dim, budget, step)
