@@ -19,35 +19,36 @@
 //                                     query g = lane % 16);
 //   softmax online per query g (lane column), rows of the S tile are tokens
 //                                     4 * (lane / 16) + i;
-//   output  O^T[d][g] += V^T[d][t] P^T[t][g]   16x16x4 fp32 MFMAs: for the
-//                                     i-th row of every lane's S tile the k
-//                                     index lane / 16 is token 4 * (lane / 16)
-//                                     + i, so the B operand is the lane's own
-//                                     probability; head_dim column m of block
-//                                     j is d = out_dim(m, j) (J = D / 16
-//                                     blocks), so the A operand is the
+//   output  O^T[d][g] += V^T[d][t] P^T[t][g]   the same MFMA over the 32
+//                                     tokens of two tiles, P split into an
+//                                     upper and a lower 16-bit part (two MFMAs
+//                                     per head_dim block): the k-slot (lane /
+//                                     16, e) is token 4 * (lane / 16) + e % 4 of
+//                                     tile e / 4, so the B operand is the
+//                                     lane's own probabilities; head_dim column
+//                                     m of block j is d = out_dim(m, j) (J = D /
+//                                     16 blocks), so the A operand is the
 //                                     elements of V's row that lane column m
 //                                     loads, and each lane ends with D / 4
 //                                     outputs of query g.
-// Probabilities stay fp32 (the reference's softmax is fp32 and multiplies
-// fp32 V).  The four waves merge in LDS.  A row that fits one span writes its
-// output directly; in a longer row every span but the last writes its
-// partial (running max, sum and unnormalised output) and exits, and the last
-// span's workgroup merges them with its own.
+// Probabilities are fp32 (the reference's softmax is fp32 and multiplies fp32
+// V) and enter the products to within 2^-14.  The four waves merge in LDS.  A
+// row that fits one span writes its output directly; in a longer row every
+// span writes its partial (running max, sum and unnormalised output, fp32)
+// with device-scope stores, waits for their acknowledgement and counts itself
+// on the row's counter, and the one that counts last merges the spans in
+// index order and resets the counter.
 //
-// Hand-over between workgroups needs no cache flushes and no counting:
-// partial values are stored as 64-bit words (tag << 32 | fp32 bits) with
-// device-scope stores, tag = launch epoch + 1, and the merging workgroup
-// re-reads (device-scope loads) any word whose tag is not yet the launch's.
-// It only waits for workgroups of lower index (the row's earlier spans),
-// which are dispatched before it, so the wait ends whether or not the grid is
-// resident at once; it is bounded all the same.  The last merging workgroup
-// advances the epoch, which keeps graph replays and workspace reuse safe.
-// The new token's K/V is read from the input rows (its working-cache slot is
-// written by the same launch), and working_lens[slot] is written by the last
-// workgroup of the row to read it, so positions may come from working_lens
-// itself.  Waits in this kernel are LDS-only barriers and the merge's tag
-// checks: the row count and the epoch load stay in flight behind the loads.
+// Every workgroup stores a "seen" word (tag << 32, tag = launch epoch + 1)
+// once it has read its position; the grid's last workgroup waits for all of
+// them, writes working_lens[slot] = position + 1 and advances the epoch,
+// which keeps graph replays and workspace reuse safe.  Positions may
+// therefore come from working_lens itself.  It only waits for workgroups of
+// lower index, which are dispatched before it, so the wait ends whether or
+// not the grid is resident at once; it is bounded all the same.  The new
+// token's K/V is read from the input rows (its working-cache slot is written
+// by the same launch).  Barriers in this kernel are LDS-only but for the wait
+// for a partial's stores: loads stay in flight behind them.
 #include "ds355_common.h"
 
 namespace ds355 {
@@ -126,13 +127,6 @@ __device__ __forceinline__ f32x4 mfma_scores<DS_FP16>(u32x4 a, u32x4 b, f32x4 c)
                                                 0, 0, 0);
 }
 
-// Element e of a packed pair word to fp32.
-template <int DT>
-__device__ __forceinline__ float unpack(uint32_t w, int half) {
-  if (DT == DS_BF16) return __uint_as_float(half ? (w & 0xffff0000u) : (w << 16));
-  return f16_to_f32(static_cast<uint16_t>(half ? (w >> 16) : (w & 0xffffu)));
-}
-
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
 // Working rows are read in whole 128-byte lines.  The A operand of the score
@@ -140,12 +134,15 @@ __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret
 // 16-byte slice quad).  Loads 2 p and 2 p + 1 of a tile therefore take line p
 // of tokens 0-7 and of tokens 8-15: lane (quad, col) holds slice quad + 4 (col
 // / 8) of token (col % 8) + 8 (i % 2), and swap_lines exchanges halves between
-// lanes col and col ^ 8.  attention_stream_kernel, whose batches come from
-// HBM, loads them non-temporally (a bare read loop on this card: 5.95 TB/s
-// cached or in half lines, 6.7-6.9 TB/s so).  A one-round batch fits the 256
-// MB last-level cache and is read again in the next draft step: cached loads
-// there (16 rows of 1987: 16.5 us, non-temporal 17.0; a 16-row draft cycle
-// 181.5 against 185.7).
+// lanes col and col ^ 8.  attention_stream_kernel loads them non-temporally
+// (a bare read loop on this card: 5.95 TB/s cached or in half lines, 6.7-6.9
+// TB/s so), also where the batch would fit the 256 MB last-level cache: four
+// draft steps over one cache that starts in HBM, us each, non-temporal /
+// cached, rows of 1987 tokens (4 heads x 128, 4 MB a row): 17 rows 22.8 / 22.8,
+// 24 23.9 / 26.3, 32 28.5 / 31.6, 48 38.4 / 42.0, 60 44.9 / 50.2 (the same cache
+// read over and over: 21.0 / 20.8, 22.4 / 23.2, 26.7 / 27.3, 36.3 / 35.8, 43.5 /
+// 42.5).  The one-shot kernel, on one round, loads them cached: 16 rows 16.3 us,
+// non-temporal 16.9; a 16-row draft cycle 180.7 against 182.2.
 constexpr int kPolicyNt = 2;
 __device__ __forceinline__ int line_token(int col, int i) { return (col & 7) + 8 * (i & 1); }
 __device__ __forceinline__ int line_elem(int quad, int col, int i) { return 8 * quad + 32 * (col >> 3) + 64 * (i >> 1); }
@@ -318,7 +315,7 @@ __device__ __forceinline__ void pair_scores(const KTiles<D>& T, const u32x4 (&qv
 // block j is out_dim(m, j), so both operands are in the lane's registers.  P
 // is split into an upper part (its fp32 value cut to the dtype) and the dtype
 // rounding of the exact remainder; two MFMAs per block keep the products
-// within ~2^-16 of fp32 probabilities.
+// within 2^-14 of fp32 probabilities (see split_prob).
 template <int DT, int D>
 __device__ __forceinline__ void pair_output(const VTiles<D>& T, const f32x4 (&sc)[2], Running<D>& run, int tb, int n,
                                             int quad, float c) {

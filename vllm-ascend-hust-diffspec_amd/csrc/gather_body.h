@@ -174,15 +174,15 @@ __device__ __forceinline__ void buf_store16(W4 v, Rsrc r, uint32_t voff, uint32_
 
 // Rows of 128 bytes (head_dim 64 in 16 bits, 32 in 32) in whole lines.  A
 // lane's two vectors of a position lie in two loads, so 4 lanes a row would
-// read and write half lines, the second half with another instruction; a
-// non-temporal half line moves whole to and from memory.  Instead lanes l and
-// l ^ 8 (positions q and q ^ 2) share the work of both positions: the lane
+// read and write half lines, the second half with another instruction, and
+// about 16% more than the rows' bytes go to memory (counters, 24 rows of
+// 130-9001 tokens, 8 heads x 64; whole lines: their bytes).  Instead lanes l
+// and l ^ 8 (positions q and q ^ 2) share the work of both positions: the lane
 // with bit 3 clear takes the first vector of each, the other the second, and
 // the swap brings the two vectors of its own position to each lane where a
-// rotation needs both (and back for the stores).  24 rows of 130-9001 tokens
-// (8 heads x 64, fp16): 39.9 -> 34.6 us together with one round of heads per
-// task (gather_wave_kernel); 24 x 8000 48.5 with neither, 46.8 with the heads
-// alone, 42.5 with both.
+// rotation needs both (and back for the stores).  Those rows (fp16): 39.9 ->
+// 34.6 us together with one round of heads per task (gather_wave_kernel); 24 x
+// 8000 48.5 with neither, 46.8 with the heads alone, 42.5 with both.
 constexpr int kRowRor8 = 0x128;  // DPP: lane c of a 16-lane row reads lane c ^ 8
 __device__ __forceinline__ uint32_t from_lane8(uint32_t own, uint32_t other, int keep_low) {
   // Lanes with bit 3 set (keep_low) or clear get `other` of lane ^ 8; the rest keep `own`.

@@ -119,12 +119,12 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(const Raw16& a, const Raw16& b, 
 
 // Keys in whole 128-byte lines.  The B operand wants 64 bytes of each of 16
 // tokens (lane kgrp * 16 + col: token col, 16-byte slice kgrp), so one load
-// per MFMA step reads half a line of every token, and a non-temporal load
-// then fetches each line twice.  Instead a pair of loads takes 128 bytes of
-// tokens 0-7 (lanes col < 8 slice kgrp, lanes col >= 8 slice 4 + kgrp of
-// token col - 8) and of tokens 8-15, and swap_lines exchanges the halves
-// between lanes col and col ^ 8: 12 VALU instructions per 2 KB, the operands
-// and so the results of the plain loads.  A bare read loop over 512 MB with
+// per MFMA step reads half a line of every token: no faster non-temporally
+// (4% more bytes fetched, by the counters).  Instead a pair of loads takes
+// 128 bytes of tokens 0-7 (lanes col < 8 slice kgrp, lanes col >= 8 slice 4 +
+// kgrp of token col - 8) and of tokens 8-15, and swap_lines exchanges the
+// halves between lanes col and col ^ 8: 12 VALU instructions per 2 KB, the
+// operands and so the results of the plain loads.  A bare read loop over 512 MB with
 // this address pattern: 5.8 TB/s cached, 6.65-6.8 non-temporal; the half-line
 // pattern 5.95 either way; contiguous 1 KB loads 6.0 and 6.8.  The steps with
 // it: 4 rows of 128k tokens 115.8 -> 100.2 us, 64 rows of 2-40k (64/8 heads)
