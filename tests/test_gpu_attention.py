@@ -272,7 +272,7 @@ def test_random_rows_positions_and_groups(cuda, seed):
 
 
 @pytest.mark.parametrize("dim", [64, 128, 256])
-@pytest.mark.parametrize("rows", [16, 320])
+@pytest.mark.parametrize("rows", [16, 400])
 def test_rows_that_end_inside_a_tile(cuda, dim, rows):
     """Row ends at and beside the half tiles (8 tokens) that key loads take lines of, in the
     one-shot kernel and (many rows) the streamed one."""
@@ -358,7 +358,7 @@ def test_expired_wait_keeps_the_working_lengths(cuda, rows, dim, budget):
 
 @pytest.mark.parametrize("rows,budget,inside", [
     (6, 512, [8, 14, 15, 16, 25, 30]),  # one-shot: the first tile pair of each wave's four
-    (40, 2048, [8, 14, 15, 16, 25, 30, 31, 40, 47, 48, 60, 63])])  # streamed
+    (50, 2048, [8, 14, 15, 16, 25, 30, 31, 40, 47, 48, 60, 63])])  # streamed
 @pytest.mark.parametrize("dim", [64, 128, 256])
 def test_infinite_value_of_the_new_token(cuda, rows, budget, inside, dim):
     """An infinity in the new token's value stays that infinity in its output column, wherever the
@@ -461,7 +461,7 @@ def test_streamed_and_one_shot_launches_share_a_workspace(cuda):
         assert _launched_streamed(dev.ws, len(slots), 4, 8, 128, 2048, n) == expect
 
 
-@pytest.mark.parametrize("rows", [3, 40])
+@pytest.mark.parametrize("rows", [3, 50])
 @pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
 def test_strided_rows_and_heads(cuda, rows, dim, dtype):
     """Queries, keys and values that are parts of one packed buffer and an output with spare
@@ -485,7 +485,7 @@ def test_strided_rows_and_heads(cuda, rows, dim, dtype):
         attention.draft_linear_attention(*args, out, dev.k, dev.v, dev.lens, list(range(rows)), None,
                                          scale=dim ** -0.5, workspace=dev.ws)
         results.append((out.cpu(), dev.k.cpu(), dev.v.cpu(), dev.lens.cpu()))
-        assert _launched_streamed(dev.ws, rows, hkv, hq // hkv, dim, budget, 1) == (rows == 40)
+        assert _launched_streamed(dev.ws, rows, hkv, hq // hkv, dim, budget, 1) == (rows == 50)
     for a, b in zip(*results):
         _same_bits(a, b)
     outside = wide.cpu()

@@ -821,10 +821,11 @@ struct StreamShape {
   // streamed, at 512 spans of head_dim 128: 16.6 / 17.2 (16 rows of 1987
   // tokens), 14.4 / 17.2 (64 rows of 184-487); 576: 21.8 / 22.5; 768: 26.9 /
   // 24.1 (1987 tokens), 22.7 / 17.9 (100-1987).  Head_dim 64, 1152 spans:
-  // 19.9 / 22.5 (36 x 1987); 1280: 18.9 / 18.3 (100-1987); 1536: 26.0 / 26.6
-  // (1987); 4096: 53.3 / 41.1 (1000-1987).  Head_dim 256, 320 spans: 21.5 /
-  // 20.7; 576: 28.5 / 27.7; 1024: 43.5 / 32.5.
-  static constexpr int kOneRound = D == 64 ? 1152 : (D == 128 ? 576 : 256);
+  // 19.9 / 22.5 (36 x 1987); 1280: 18.9 / 18.3 (100-1987), 22.6 / 23.9 (20 x
+  // 4032); 1472: 26.1 / 26.7; 1536: 26.4 / 26.6 (1987); 1792: 30.2 / 28.0; 4096:
+  // 53.3 / 41.1 (1000-1987).  Head_dim 256, 320 spans: 21.5 / 20.7; 384: 18.0 /
+  // 19.3 (12 x 950), 27.4 / 24.9 (3 x 4032); 576: 28.5 / 27.7; 1024: 43.5 / 32.5.
+  static constexpr int kOneRound = D == 64 ? 1536 : (D == 128 ? 576 : 256);
 };
 
 struct Ranges {  // workgroup w < used takes spans [start(w), start(w + 1))
